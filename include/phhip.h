@@ -376,9 +376,10 @@ int ph_reduce2d_all(const ph_prog *prog, int32_t n_in, const void *const *ins,
  * is Float64).  dtype PH_F32, the build's own Float32 variant, computes the
  * last multiply and add with one rounding, u' = fma(d, r, u); its accuracy
  * is stated against the Float64 run.  u holds the initial field and
- * receives the final one; tmp is scratch of the same size.  Up to eight
- * (Float64) or twelve (Float32) steps run per pass over the grid (temporal
- * blocking), bit-identical to single steps.  If
+ * receives the final one; tmp is scratch of the same size.  Many steps
+ * run per pass over the grid (tiles of it stay in registers meanwhile; a grid
+ * of up to 64 x 64 cells runs them all in one launch), bit-identical to single
+ * steps.  If
  * energy_every > 0, energy_out
  * (device, steps/energy_every + 1 doubles) receives the FP64 sum of u at
  * steps 0, energy_every, 2*energy_every, ...
@@ -392,8 +393,8 @@ int ph_heat2d(int32_t dtype, void *u, void *tmp, int64_t ny, int64_t nx,
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments and the same results, bit for bit.  ph_heat2d keeps the partial
  * sums of its FP64 energy reductions in library scratch that grows on
- * demand; this variant keeps them in a fixed 32 KiB device array (2048
- * groups, the most the reduction uses for any grid), whose address ph_init
+ * demand; this variant keeps them in a fixed 256 KiB device array (two
+ * sums of 8192 groups, the most a pass leaves), whose address ph_init
  * looks up on its device, and it skips ph_heat2d's one read-back of max|u|
  * (the fused first operation it enables changes no result).  Every call on a
  * device shares that array, and each reduction writes every slot it later
