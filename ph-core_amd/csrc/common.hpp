@@ -58,6 +58,11 @@ struct Layout {
   int64_t offset[kMaxOps];
   int64_t stride[kMaxOps][PH_MAX_RANK];
 };
+inline int64_t layout_count(const Layout &L) {
+  int64_t n = 1;
+  for (int k = 0; k < L.rank; ++k) n *= L.shape[k];
+  return n;
+}
 // All descriptors must be affine (nstage == 0) with equal logical shapes.
 void collapse(const ph_view_desc *const *descs, int nops, Layout *out);
 
