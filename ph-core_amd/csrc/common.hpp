@@ -25,11 +25,16 @@ int device();
 
 // Lazily grown device scratch, valid until the next call that asks for more;
 // all work on it is ordered by the single library stream.  Slots: 0-1
-// gathered map and reduction inputs, 2 reduction and heat partials, 3 flag
-// words, 4-7 the buffers of maps whose inputs share the output's buffer,
+// gathered map and reduction inputs, 2 reduction and heat partials, 3 ordered
+// maps' words, 4-7 the buffers of maps whose inputs share the output's buffer,
 // 8 the inverse of an indexed map's write index, 9-11 the marks, depths and
 // level counts of an ordered map's tree of dependents.
 int scratch(size_t bytes, void **out, int slot = 0);
+
+// Copies device memory to the host and waits for the stream; up to
+// kFetchBytes go through a page the library keeps (under the ABI lock).
+constexpr size_t kFetchBytes = size_t(1) << 16;
+int fetch(void *dst, const void *src, size_t bytes);
 
 // ph_strided_copy when source and destination share a buffer: the copy in
 // the reference's lexicographic order (each element read after the writes

@@ -412,6 +412,17 @@ __device__ __forceinline__ float ph_pow(float a, float b) { return __builtin_pow
 __device__ __forceinline__ double ph_pow(double a, double b) { return __builtin_pow(a, b); }
 __device__ __forceinline__ float ph_fmod_floor(float a, float b) { const float q = __builtin_floorf(a / b); const float m = b * q; return a - m; }
 __device__ __forceinline__ double ph_fmod_floor(double a, double b) { const double q = __builtin_floor(a / b); const double m = b * q; return a - m; }
+// Raises flag bits: the first raise of a bit stores 1 into its host word (the
+// block: guard word, reduction ticket, address of the host words).
+__device__ __forceinline__ void ph_raise(int *f, int fl) {
+  if (fl == 0) return;
+  if (!(fl & ~__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) return;
+  const int fresh = fl & ~atomicOr(f, fl);
+  if (fresh == 0) return;
+  int *h = *(int **)(f + 2);
+  for (int k = 0; k < 3; ++k)
+    if (fresh >> k & 1) __hip_atomic_store(h + k, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 template <typename F> __device__ __forceinline__ F ph_powi(F a, int b) {
   const bool recip = b < 0; long long e = b; if (e < 0) e = -e; F r = (F)1;
   for (;;) { if (e & 1) r *= a; e /= 2; if (e == 0) break; a *= a; }
@@ -582,7 +593,7 @@ std::string map_source(const ph_prog *p, int n_in, const int *in_dt, const ph::L
              lit_i64(inner_stride(n_in)).c_str(), res0.c_str());
     s += "      }\n    }\n  }\n";
   }
-  s += "  if (fl) atomicOr(A.flags, fl);\n}\n";
+  s += "  ph_raise(A.flags, fl);\n}\n";
   return s;
 }
 
@@ -690,7 +701,7 @@ std::string map_tiled_source(const ph_prog *p, int n_in, const int *in_dt, const
   s += fmt("          ph_st((%s *)A.out, base%d + aa * %s + bc * %s, %s);\n", stype(out_dt), n_in,
            lit_i64(L.stride[n_in][ax]).c_str(), lit_i64(L.stride[n_in][bx]).c_str(), res.c_str());
   s += "        }\n      }\n    }\n    __syncthreads();  // the next tile reuses the LDS\n  }\n";
-  s += "  if (fl) atomicOr(A.flags, fl);\n}\n";
+  s += "  ph_raise(A.flags, fl);\n}\n";
   return s;
 }
 
@@ -722,29 +733,57 @@ int64_t grid_for(int64_t blocks) {
   return blocks < 1 ? 1 : (blocks > cap ? cap : blocks);
 }
 
-// The flag word is cleared by a one-thread kernel (not a memset node, so the
-// sequence stays valid inside a captured HIP graph) and read back only when
-// the program contains an operation that can raise a flag.
-int get_flags_buffer(int **dflags, bool clear) {
-  void *p;
-  int rc = ph::scratch(64, &p, 3);
-  if (rc) return rc;
-  *dflags = (int *)p;
-  if (clear) return ph::clear_i32(*dflags, 1);
+// Flags of maps and reductions.  A kernel that raises a bit for the first time
+// stores into a word of coherent host memory (ph_raise in the prelude), so the
+// usual call, which raises nothing, needs neither a clearing kernel before nor
+// a copy back after it: only the wait for the stream, which the caller's
+// exception requires.  (Two checked operators on a 32 x 48 Int32 array took 58
+// us with a clear, a copy and a wait each.)  Guard and host words are zero
+// between calls: read_flags clears what a call raised, under the ABI lock.  A
+// call without flags_out raises into a block of its own that is never read.
+struct FlagBlock {
+  int *dev = nullptr;   // guard, ticket, address of the host words
+  int *host = nullptr;  // one word per bit
+};
+constexpr int kFlagBits = 3;
+
+int *g_flag_host = nullptr;  // the host words of the block that is read
+
+int get_flags_buffer(int **dflags, bool wanted) {
+  static FlagBlock blocks[2];  // read, never read
+  FlagBlock &b = blocks[wanted ? 0 : 1];
+  if (!b.dev) {
+    int *host = nullptr, *dev = nullptr;
+    PH_HIP(hipHostMalloc((void **)&host, 64, hipHostMallocCoherent));
+    std::memset(host, 0, 64);
+    if (hipMalloc((void **)&dev, 64) != hipSuccess) {
+      (void)hipHostFree(host);
+      return ph::set_error(PH_E_OOM, "flag words");
+    }
+    int init[16] = {0};
+    std::memcpy(init + 2, &host, sizeof(host));
+    PH_HIP(hipMemcpyAsync(dev, init, 64, hipMemcpyHostToDevice, ph::stream()));
+    PH_HIP(hipStreamSynchronize(ph::stream()));
+    b.dev = dev;
+    b.host = host;
+  }
+  if (wanted) g_flag_host = b.host;
+  *dflags = b.dev;
   return PH_OK;
 }
 
 int read_flags(int *dflags, bool may_flag, int32_t *flags_out) {
   if (!flags_out) return PH_OK;
-  if (!may_flag) {
-    *flags_out = 0;
-    return PH_OK;
-  }
-  int v = 0;
-  PH_HIP(hipMemcpyAsync(&v, dflags, sizeof(int), hipMemcpyDeviceToHost, ph::stream()));
+  *flags_out = 0;
+  if (!may_flag) return PH_OK;
   PH_HIP(hipStreamSynchronize(ph::stream()));
-  *flags_out = v;
-  return PH_OK;
+  volatile int *h = g_flag_host;
+  for (int k = 0; k < kFlagBits; ++k)
+    if (h[k]) {
+      *flags_out |= 1 << k;
+      h[k] = 0;
+    }
+  return *flags_out ? ph::clear_i32(dflags, 1) : PH_OK;
 }
 
 // Compiled fused kernels, keyed by everything their source depends on (the
@@ -1291,7 +1330,7 @@ std::string red_tile_float(const ph_prog *p, int n_in, const int *in_dt, const i
     s += "    for (int w = 1; w < 4; ++w) { S b; st_from(b, rsum_sh[i][w], (double)rmax_sh[i][w]); a = st_comb(a, b); }\n";
     s += fmt("    ((S *)A.rowpart)[ct * %s + r0 + i] = a;\n  }\n", lit_i64(P.rows).c_str());
   }
-  s += "  if (fl) atomicOr(A.flags, fl);\n}\n";
+  s += "  ph_raise(A.flags, fl);\n}\n";
   return s;
 }
 
@@ -1368,7 +1407,7 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
     s += "    S a = rowsh[i][0]; a = st_comb(a, rowsh[i][1]); a = st_comb(a, rowsh[i][2]); a = st_comb(a, rowsh[i][3]);\n";
     s += fmt("    ((S *)A.rowpart)[ct * %s + r0 + i] = a;\n  }\n", lit_i64(P.rows).c_str());
   }
-  s += "  if (fl) atomicOr(A.flags, fl);\n}\n";
+  s += "  ph_raise(A.flags, fl);\n}\n";
   }
   if ((P.do_rows && P.ntc > kRowFold) || (P.do_cols && P.ntr > kRowFold)) {
     // pre-fold: state t of series i (a row over its column tiles, or a column
@@ -1557,7 +1596,7 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
       }
     }
   }
-  s += "  }\n  if (fl) atomicOr(A.flags, fl);\n}\n";
+  s += "  }\n  ph_raise(A.flags, fl);\n}\n";
   return s;
 }
 
@@ -1708,7 +1747,7 @@ int run_reduce2d(const ph_prog *prog, int n_in, const void *const *ins, const in
                    &base, 2);
   if (rc) return rc;
   int *dflags;
-  rc = get_flags_buffer(&dflags, may_flag);
+  rc = get_flags_buffer(&dflags, flags_out != nullptr);
   if (rc) return rc;
   RedArgs A;
   std::memset(&A, 0, sizeof(A));
@@ -1817,7 +1856,7 @@ int map_tiled(const ph_prog *prog, int n_in, const void *const *ins, const int *
   }
   const bool may_flag = prog_may_flag(prog);
   int *dflags;
-  int rc = get_flags_buffer(&dflags, may_flag);
+  int rc = get_flags_buffer(&dflags, flags_out != nullptr);
   if (rc) return rc;
   MapArgs A;
   std::memset(&A, 0, sizeof(A));
@@ -3286,7 +3325,7 @@ int ph_map(const ph_prog *prog, int32_t n_in, const void *const *ins, const ph_v
   }
   const bool may_flag = prog_may_flag(prog);
   int *dflags;
-  rc = get_flags_buffer(&dflags, may_flag);
+  rc = get_flags_buffer(&dflags, flags_out != nullptr);
   if (rc) return rc;
   MapArgs A;
   std::memset(&A, 0, sizeof(A));

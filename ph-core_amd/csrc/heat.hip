@@ -197,8 +197,8 @@ int fused_safe(const T *u, int64_t n, T r, bool *safe, int64_t *steps_ok) {
   rc = ph::check_launch("k_absmax_bits");
   if (rc) return rc;
   U m = 0;
-  PH_HIP(hipMemcpyAsync(&m, p, sizeof(U), hipMemcpyDeviceToHost, ph::stream()));
-  PH_HIP(hipStreamSynchronize(ph::stream()));
+  rc = ph::fetch(&m, p, sizeof(U));
+  if (rc) return rc;
   *safe = m <= Bits<T>::kLimit;
   *steps_ok = (int64_t)(0.5 * std::log(4.0) / (11.0 * Bits<T>::kEps));
   return PH_OK;

@@ -61,6 +61,37 @@ int scratch(size_t bytes, void **out, int slot) {
   return PH_OK;
 }
 
+// Copies small results to the host through a page of coherent host memory that
+// a kernel writes: the runtime's own copy to pageable memory stages them as
+// well, at several times the overhead.
+static __global__ void k_to_host(char *__restrict__ dst, const char *__restrict__ src, unsigned bytes) {
+  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x, n = gridDim.x * blockDim.x;
+  const bool words = ((uintptr_t)src & 7) == 0;
+  const unsigned whole = words ? bytes / 8 : 0;
+  for (unsigned i = t; i < whole; i += n) ((uint64_t *)dst)[i] = ((const uint64_t *)src)[i];
+  for (unsigned i = whole * 8 + t; i < bytes; i += n) dst[i] = src[i];
+}
+
+int fetch(void *dst, const void *src, size_t bytes) {
+  static void *page = nullptr;
+  if (bytes <= kFetchBytes && !page && hipHostMalloc(&page, kFetchBytes, hipHostMallocCoherent) != hipSuccess) {
+    page = nullptr;
+    (void)hipGetLastError();
+  }
+  if (bytes <= kFetchBytes && page) {
+    const unsigned groups = (unsigned)((bytes + 2047) / 2048);
+    hipLaunchKernelGGL(k_to_host, dim3(groups), dim3(256), 0, g_stream, (char *)page, (const char *)src, (unsigned)bytes);
+    int rc = check_launch("k_to_host");
+    if (rc) return rc;
+    PH_HIP(hipStreamSynchronize(g_stream));
+    std::memcpy(dst, page, bytes);
+    return PH_OK;
+  }
+  PH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, g_stream));
+  PH_HIP(hipStreamSynchronize(g_stream));
+  return PH_OK;
+}
+
 size_t dtype_size(int dt) {
   switch (dt) {
     case PH_I32: return 4;
@@ -265,9 +296,7 @@ int ph_d2h(void *dst, const void *src, size_t bytes) {
   PH_GUARD();
   PH_REQUIRE_INIT();
   if (bytes == 0) return PH_OK;
-  PH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ph::g_stream));
-  PH_HIP(hipStreamSynchronize(ph::g_stream));
-  return PH_OK;
+  return ph::fetch(dst, src, bytes);
 }
 
 int ph_d2d(void *dst, const void *src, size_t bytes) {
