@@ -1096,16 +1096,24 @@ struct RedPlan {
   bool colex = false;  // the view's lexicographic order runs down the columns (a swapped transposed view)
   int64_t ntc_fin = 0;  // column-tile states per row left for the finish after the pre-folds
   int64_t ntr_fin = 0;  // row-tile states per column, likewise
+  int parts = 4;        // threads that fold one column's states in the finish (256 / parts columns a block)
 };
 
 // Column-tile states per row that the finish folds on one thread; rows with
-// more are pre-folded in ordered runs of this many (ph_red_prefold), and so
-// are the row-tile states of columns with more.
+// more are pre-folded in ordered runs of this many (ph_red_prefold).  A
+// column's row-tile states are folded by 4 threads, or by 16 where there are
+// enough of them to share and blocks of 64 columns would not fill the CUs, and
+// are pre-folded beyond 16 each.  Four threads, and a pre-fold beyond 64 states,
+// took 6 us more of 18-35 us: Float32 3000^2 24.7 -> 18.2 us, 2048^2 18.3 ->
+// 12.7, BFloat16 5003 x 3001 34.8 -> 28.7, 4096 x 40 17.1 -> 12.6; at 16384
+// columns the two measure alike.
 constexpr int64_t kRowFold = 64;
-int64_t prefolded(int64_t ntc) {
-  while (ntc > kRowFold) ntc = (ntc + kRowFold - 1) / kRowFold;
+constexpr int64_t kColFold = 256;
+int64_t prefolded(int64_t ntc, int64_t most) {
+  while (ntc > most) ntc = (ntc + kRowFold - 1) / kRowFold;
   return ntc;
 }
+int column_parts(int64_t ntr_fin, int64_t cols) { return ntr_fin > 64 || (ntr_fin > 16 && cols < 256 * 64) ? 16 : 4; }
 
 // Offset of column C (an i64 expression) of input j.
 std::string col_offset(const RedPlan &P, const int64_t *cs, int j, const std::string &C) {
@@ -1492,7 +1500,7 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
   }
   s += "  ph_raise(A.flags, fl);\n}\n";
   }
-  if ((P.do_rows && P.ntc > kRowFold) || (P.do_cols && P.ntr > kRowFold)) {
+  if ((P.do_rows && P.ntc > kRowFold) || (P.do_cols && P.ntr > kColFold)) {
     // pre-fold: state t of series i (a row over its column tiles, or a column
     // over its row tiles) <- the states [t * 64, t * 64 + 64) of the level
     // below, in order (a long series would otherwise be folded on one or four
@@ -1507,12 +1515,13 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
     s += "  S a; st_init(a);\n#pragma unroll 8\n  for (i64 u = t0; u < t1; ++u) a = st_comb(a, ((const S *)F.src)[u * F.rows + i]);\n";
     s += "  ((S *)F.dst)[t * F.rows + i] = a;\n}\n";
   }
-  // --- finish.  Column blocks: 64 columns x 4 parts; part p folds row tiles
-  // [p*ntr/4, (p+1)*ntr/4) in order, then the 4 parts are folded in order.
+  // --- finish.  Column blocks: 64 columns x 4 parts (or 16 x 16); part p folds
+  // row tiles [p*ntr/4, (p+1)*ntr/4) in order, then the parts are folded in order.
   // Row blocks: one row per thread (its column tiles in order), then the
   // block's 256 rows are folded in order (a pairwise tree of adjacent
   // ranges) into one state per block for the full result.
-  const int64_t ncb = P.do_cols ? (P.cols + 63) / 64 : 0;
+  const int fc = 256 / P.parts;
+  const int64_t ncb = P.do_cols ? (P.cols + fc - 1) / fc : 0;
   const bool fix = std::string(P.state) != "SI";  // float maxima follow Enumerable#max's `>`
   auto ovf = [&](const char *st) {
     // (a sum outside Int32 is an overflow whatever the bounds say)
@@ -1524,10 +1533,10 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
   s += "  __shared__ S sh[256];\n  int fl = 0;\n";
   if (P.do_cols) {
     s += fmt("  if ((i64)blockIdx.x < %s) {\n", lit_i64(ncb).c_str());
-    s += "    const int lane = threadIdx.x & 63; const int part = threadIdx.x >> 6;\n";
-    s += "    const i64 c = (i64)blockIdx.x * 64 + lane;\n";
-    s += fmt("    const i64 t0 = part * %s / 4, t1 = (part + 1) * %s / 4;\n", lit_i64(P.ntr_fin).c_str(),
-             lit_i64(P.ntr_fin).c_str());
+    s += fmt("    const int lane = threadIdx.x & 63; const int part = threadIdx.x / %d;\n", fc);
+    s += fmt("    const i64 c = (i64)blockIdx.x * %d + threadIdx.x %% %d;\n", fc, fc);
+    s += fmt("    const i64 t0 = part * %s / %d, t1 = (part + 1) * %s / %d;\n", lit_i64(P.ntr_fin).c_str(), P.parts,
+             lit_i64(P.ntr_fin).c_str(), P.parts);
     s += "    S a; st_init(a);\n";
     if (fix) {
       // the column's first element, loaded before the fold so its latency overlaps it
@@ -1537,7 +1546,7 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
     }
     // (the states are loaded eight at a time before they are folded in
     // order, so the loads of a group are in flight together)
-    const int64_t per = (P.ntr_fin + 3) / 4;
+    const int64_t per = (P.ntr_fin + P.parts - 1) / P.parts;
     s += fmt("    if (c < %s) {\n#pragma unroll\n      for (int g = 0; g < %s; g += 8) {\n        S v[8];\n"
              "#pragma unroll\n        for (int u = 0; u < 8; ++u) {\n"
              "          const i64 t = t0 + g + u;\n          if (g + u < %s && t < t1) v[u] = ((const S *)A.colpart)[t * %s + c];\n        }\n"
@@ -1550,14 +1559,14 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
       // greater: a leading NaN stays, and of equal zeros the first one's
       // sign.  Columns whose maximum is a zero are scanned by the whole
       // wavefront in turn, 64 rows at a time, for their first zero.
-      s += "    if (part == 0) {\n      double mx = 0.0;\n      bool mzero = false;\n";
-      s += fmt("      if (c < %s) {\n", lit_i64(P.cols).c_str());
-      s += "        S r = sh[lane];\n        for (int q = 1; q < 4; ++q) r = st_comb(r, sh[q * 64 + lane]);\n";
+      s += "    if (threadIdx.x < 64) {\n      double mx = 0.0;\n      bool mzero = false;\n";
+      s += fmt("      const bool mine = part == 0 && c < %s;\n      if (mine) {\n", lit_i64(P.cols).c_str());
+      s += fmt("        S r = sh[lane];\n        for (int q = 1; q < %d; ++q) r = st_comb(r, sh[q * %d + lane]);\n", P.parts, fc);
       s += "        if (A.col_sum) { A.col_sum[c] = st_sum(r); " + ovf("r") + " }\n";
       s += "        mx = st_max(r);\n        mzero = A.col_max && f0 == f0 && mx == 0.0;\n      }\n";
       s += "      unsigned long long need = __ballot(mzero);\n";
       s += "      while (need) {\n        const int l = __builtin_ctzll(need);\n        need &= need - 1;\n";
-      s += "        const i64 cl = (i64)blockIdx.x * 64 + l;\n";
+      s += fmt("        const i64 cl = (i64)blockIdx.x * %d + l;\n", fc);
       s += fmt("        bool found = false;\n        for (i64 r1 = 0; r1 < %s && !found; r1 += 512) {\n          double g[8];\n"
                "#pragma unroll\n          for (int k = 0; k < 8; ++k) {\n            const i64 rr = r1 + 64 * k + lane;\n"
                "            g[k] = 1.0;\n            if (rr < %s) {\n", lit_i64(P.rows).c_str(), lit_i64(P.rows).c_str());
@@ -1570,11 +1579,10 @@ std::string red_source(const ph_prog *p, int n_in, const int *in_dt, const int64
       s += "            const unsigned long long hit = __ballot(g[k] == 0.0);\n            if (hit && !found) {\n";
       s += "              const double gz = __shfl(g[k], __builtin_ctzll(hit));\n";
       s += "              if (lane == l) mx = gz;\n              found = true;\n            }\n          }\n        }\n      }\n";
-      s += fmt("      if (c < %s && A.col_max) {\n        if (f0 != f0) mx = f0;\n        A.col_max[c] = mx;\n      }\n",
-               lit_i64(P.cols).c_str());
+      s += "      if (mine && A.col_max) {\n        if (f0 != f0) mx = f0;\n        A.col_max[c] = mx;\n      }\n";
     } else {
       s += fmt("    if (part == 0 && c < %s) {\n", lit_i64(P.cols).c_str());
-      s += "      S r = sh[lane];\n      for (int q = 1; q < 4; ++q) r = st_comb(r, sh[q * 64 + lane]);\n";
+      s += fmt("      S r = sh[lane];\n      for (int q = 1; q < %d; ++q) r = st_comb(r, sh[q * %d + lane]);\n", P.parts, fc);
       s += "      if (A.col_sum) { A.col_sum[c] = st_sum(r); " + ovf("r") + " }\n";
       s += "      if (A.col_max) A.col_max[c] = st_max(r);\n";
     }
@@ -1780,7 +1788,7 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
                   ((uintptr_t)ins[j] % align) == 0;
   }
   P.ntc = (P.cols + 256 * P.vec - 1) / (256 * P.vec);
-  P.ntc_fin = prefolded(P.ntc);
+  P.ntc_fin = prefolded(P.ntc, kRowFold);
   // rows per tile: aim for ~512 workgroups (fewer, taller tiles write fewer
   // column partial states; measured best on 16384^2), a multiple of 16 (the
   // float tile folds rows 8 at a time), at most 1024 rows (256 for integer
@@ -1795,7 +1803,8 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
   if (tr < 1) tr = 1;
   P.tr = (int)tr;
   P.ntr = (P.rows + P.tr - 1) / P.tr;
-  P.ntr_fin = prefolded(P.ntr);
+  P.ntr_fin = prefolded(P.ntr, kColFold);
+  P.parts = column_parts(P.ntr_fin, P.cols);
   std::string key = "R" + prog_key(prog);
   key_add(&key, in_dt, sizeof(int) * (size_t)n_in);
   key_add(&key, V.rs, sizeof(int64_t) * (size_t)n_in);
@@ -1806,7 +1815,7 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
   if (P.cols2) key_add(&key, P.cs2, sizeof(int64_t) * (size_t)n_in);
   key += P.state;
   hipFunction_t ktile, kfin, kfold = nullptr;
-  const bool fold_rows = P.do_rows && P.ntc > kRowFold, fold_cols = P.do_cols && P.ntr > kRowFold;
+  const bool fold_rows = P.do_rows && P.ntc > kRowFold, fold_cols = P.do_cols && P.ntr > kColFold;
   const bool prefold = fold_rows || fold_cols;
   int rc;
   auto hit = fused_cache().find(key);
@@ -1871,7 +1880,7 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
   // ordered pre-folds of long series of tile states, 64 to 1, ping-pong
   // between the tile kernel's buffer and a fold buffer, until the finish's
   // count is left; returns the buffer holding the last level
-  auto fold = [&](void *states, char *spare, int64_t series, int64_t n) -> void * {
+  auto fold = [&](void *states, char *spare, int64_t series, int64_t n, int64_t most) -> void * {
     struct {
       const void *src;
       void *dst;
@@ -1879,7 +1888,7 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
     } F;
     char *lv[2] = {(char *)states, spare};
     int cur = 0;
-    while (n > kRowFold) {
+    while (n > most) {
       const int64_t nout = (n + kRowFold - 1) / kRowFold;
       F.src = lv[cur];
       F.dst = lv[cur ^ 1];
@@ -1897,12 +1906,13 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
     return lv[cur];
   };
   char *spare = (char *)A.rowzero + al(rowzero_b);
-  if (fold_rows && !(A.rowpart = fold(A.rowpart, spare, P.rows, P.ntc)))
+  if (fold_rows && !(A.rowpart = fold(A.rowpart, spare, P.rows, P.ntc, kRowFold)))
     return ph::set_error(PH_E_HIP, "reduction pre-fold launch failed");
-  if (fold_cols && !(A.colpart = fold(A.colpart, spare + al(fold_b), P.cols, P.ntr)))
+  if (fold_cols && !(A.colpart = fold(A.colpart, spare + al(fold_b), P.cols, P.ntr, kColFold)))
     return ph::set_error(PH_E_HIP, "reduction pre-fold launch failed");
-  // finish: column blocks of 64 columns, then row blocks of 256 rows
-  const int64_t nfin = (P.do_cols ? (P.cols + 63) / 64 : 0) + (P.do_rows ? (P.rows + 255) / 256 : 0);
+  // finish: column blocks of 256 / parts columns, then row blocks of 256 rows
+  const int64_t fc = 256 / P.parts;
+  const int64_t nfin = (P.do_cols ? (P.cols + fc - 1) / fc : 0) + (P.do_rows ? (P.rows + 255) / 256 : 0);
   if (nfin > 0)
     PH_HIP(hipModuleLaunchKernel(kfin, (unsigned)nfin, 1, 1, 256, 1, 1, 0, ph::stream(), nullptr, cfg));
   return read_flags(dflags, may_flag, flags_out);
@@ -3245,10 +3255,11 @@ int ph_compile_check(const ph_prog *prog, int32_t n_in, const int32_t *in_dtypes
   P.vec = red_vec(std::string(P.state) == "SI", n_in, in_dt);
   for (int j = 0; j < PH_MAX_INPUTS; ++j) P.vec_ok[j] = j < n_in && cols % P.vec == 0;
   P.ntc = (cols + 256 * P.vec - 1) / (256 * P.vec);
-  P.ntc_fin = prefolded(P.ntc);
+  P.ntc_fin = prefolded(P.ntc, kRowFold);
   P.tr = 64;
   P.ntr = (rows + 63) / 64;
-  P.ntr_fin = prefolded(P.ntr);
+  P.ntr_fin = prefolded(P.ntr, kColFold);
+  P.parts = column_parts(P.ntr_fin, cols);
   return ph::jit_compile_only(red_source(prog, n_in, in_dt, V.rs, V.cs, P));
 }
 
