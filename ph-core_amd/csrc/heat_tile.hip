@@ -23,10 +23,12 @@
 // additions) and 8.1 at Float64 (six, and two shifts of two words each per
 // pair of cells).  At 8192^2 that keeps the vector ALUs 96% busy at Float32;
 // the rest is the overlap (a third of the cells at 16 steps and 128 x 256).
-// Time per step, the sweep's and this kernel's, passes only:
-//   8192^2     Float32 14.7 -> 14.3 us, Float64 33 -> 27.5 us
-//   1024^2     Float64 5.1 -> 1.24 us
-//   750 x 1111 Float64 4.5 -> 1.18 us
+// Time per step, the sweep's and this kernel's, over runs of 100 steps (passes
+// of at most two steps may lose: Float32 8192^2 59 -> 62 us, 5000 x 7000 31 -> 35):
+//   8192^2     Float32 18.5 -> 14.2 us, Float64 36 -> 27.4 us
+//   2048^2     Float32 3.9 -> 1.58, Float64 5.6 -> 3.0 us
+//   1024^2     Float32 3.6 -> 0.89, Float64 3.9 -> 1.27 us
+//   750 x 1111 Float32 6.1 -> 0.88, Float64 5.8 -> 1.18 us
 //   64^2       Float64 2.7 -> 0.41 us (one workgroup)
 //
 // Every cell is computed with the single-step formula, so results are
@@ -64,7 +66,15 @@ __global__ __launch_bounds__(64 * W) void k_heat_tile(const T *u, T *out, TileAr
   __shared__ T sh[2][W + 2][2][TX];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int64_t tx = (int)blockIdx.x % a.ntx, ty = (int)blockIdx.x / a.ntx;
+  // Each XCD (workgroups are dealt to the eight in turn) takes an eighth of the
+  // tiles in order, so that its L2 sees both writers of a line and the overlap
+  // that neighbours read (8192^2 one step, with vector stores below, against
+  // tiles dealt in turn: Float32 147 -> 114 us, Float64 254 -> 199; 16 and 10
+  // steps a pass: 14.6 -> 14.2 and 28.1 -> 27.4 us a step, 1024^2 1.19 -> 0.89
+  // and 1.51 -> 1.27).
+  const int q8 = (int)gridDim.x >> 3, r8 = (int)gridDim.x & 7, xcd = (int)blockIdx.x & 7;
+  const int tile = xcd * q8 + (xcd < r8 ? xcd : r8) + ((int)blockIdx.x >> 3);
+  const int64_t tx = tile % a.ntx, ty = tile / a.ntx;
   // the tile's first cell: `h` before the cells it writes, moved inside the
   // grid (a tile flush with an edge needs no overlap there)
   const int64_t mx = a.nx > TX ? a.nx - TX : 0, my = a.ny > TY ? a.ny - TY : 0;
@@ -162,7 +172,7 @@ __global__ __launch_bounds__(64 * W) void k_heat_tile(const T *u, T *out, TileAr
     if (threadIdx.x == 0) {
       for (int w = 1; w < W; ++w) e = d2_comb(e, esh[w]);
       if (gridDim.x == 1) *(double *)part = e.s + e.c;
-      else part[blockIdx.x] = e;
+      else part[tile] = e;
     }
     __syncthreads();
   };
@@ -205,9 +215,16 @@ __global__ __launch_bounds__(64 * W) void k_heat_tile(const T *u, T *out, TileAr
   for (int i = 0; i < R; ++i)
     if (i >= ry0 && i < ry1) {
       T *row = out + (y + i) * a.nx + xs;
+      if (own[0] && own[V - 1]) {
+        RowU t;
 #pragma unroll
-      for (int v = 0; v < V; ++v)
-        if (own[v]) row[(unsigned)(lx + v)] = c[i][v];
+        for (int v = 0; v < V; ++v) t.v[v] = c[i][v];
+        *(RowU *)(row + (unsigned)lx) = t;
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+          if (own[v]) row[(unsigned)(lx + v)] = c[i][v];
+      }
     }
 }
 
