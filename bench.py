@@ -357,7 +357,7 @@ def main():
     achieved_g = gather_bytes / (ms_gather * 1e-3) / 1e9
 
     traffic = load_traffic()
-    roofline = {"bound": "hbm", "kernel": "k_fill_scatter_vec<uint32_t,4> (fused NArray.fill + MutableView scatter)",
+    roofline = {"bound": "hbm", "kernel": "k_fill_scatter_flat<uint32_t> (fused NArray.fill + MutableView scatter)",
                 "achieved": round(achieved_fs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                 "frac": round(achieved_fs / PEAK_HBM_GBS, 4),
                 "traffic": traffic.get("k_fill_scatter") if traffic else None,
@@ -377,7 +377,7 @@ def main():
     cx = phase.NArray.random([1 << 26], D.I32, seed=9, dist="int31")
     cx.clone()
     ms_copy = time_loop(ev, lambda: cx.clone(), 10, phase)
-    extra["copy_256mib"] = {"kernel": "k_copy_rows (contiguous)", "bytes": 2 << 28, "ms_per_launch": round(ms_copy, 4),
+    extra["copy_256mib"] = {"kernel": "k_copy_flat_vec (contiguous)", "bytes": 2 << 28, "ms_per_launch": round(ms_copy, 4),
                             "achieved_gbs": round((2 << 28) / ms_copy / 1e6, 1)}
     del cx
 
@@ -489,7 +489,7 @@ def other_workloads(phase, ev, args):
         big = phase.NArray.random([1 << 29], D.I32, seed=9, dist="int31")
         big.clone()
         msb = time_loop(ev, lambda: big.clone(), 5, phase)
-        out["copy_2gib"] = {"kernel": "k_copy_rows (contiguous)", "bytes": 2 << 31, "ms": round(msb, 4),
+        out["copy_2gib"] = {"kernel": "k_copy_flat_vec (contiguous)", "bytes": 2 << 31, "ms": round(msb, 4),
                             "achieved_gbs": round((2 << 31) / msb / 1e6, 1),
                             "note": "practical HBM copy ceiling for multi-GB working sets"}
         # the runtime's own device-to-device copy of the same 2 GiB
@@ -537,7 +537,7 @@ def other_workloads(phase, ev, args):
         # the same run with 1, 2 and 4 steps per pass for both precisions (one
         # step per pass is the reference's loop structure; 1 and 2 are
         # HBM-bound in both precisions), next to
-        # the default schedule (16-17 steps per pass for FP32, 10 for FP64,
+        # the default schedule (20 steps per pass for FP32, 10 for FP64,
         # where FP32 is limited by VALU: it runs at FP64's rate without packed
         # FP32 math)
         per_pass = {}
@@ -582,8 +582,7 @@ def other_workloads(phase, ev, args):
                                                      "frac_of_roofline_f32": round(per_pass["1"]["F32"] / 1000.0, 3)},
                                "rel_l2_f32_vs_f64": rel,
                                "roofline_gcells_f64": 500.0, "roofline_gcells_f32": 1000.0,
-                               "traffic_per_launch_of_four_steps": {"f64": tr.get("k_heat_multi_f64"),
-                                                                    "f32": tr.get("k_heat_multi_f32")}}
+                               "traffic_per_pass": {"f64": tr.get("k_heat_tile_f64"), "f32": tr.get("k_heat_tile_f32")}}
         del fields, u
         if not args.no_cpu:
             out["c4_heat_8192"]["cpu"] = cpu_c4(u0)
@@ -669,7 +668,7 @@ def path_ops(phase, ev, args):
     if O:
         from crystal import parse_literal
         r = O.region([parse_literal(f"0...{rows}"), parse_literal("..")], [n, n])
-    entry("transpose_gather", "k_copy_tiled_v (LDS 128x128 tiles, 16-byte lanes)", lambda: x.view().permute(1, 0).to_narr(), 8 * nn,
+    entry("transpose_gather", "k_copy_tiled (LDS tiles, 16-byte lanes)", lambda: x.view().permute(1, 0).to_narr(), 8 * nn,
           lambda: _cpu_leg(lambda: O.view_gather(xh, [("region", r), ("permute", [1, 0])], [rows, n]),
                            8 * rows * n, "view_gather of x.permute(1, 0)", f"its first {rows} rows"))
     zt = z.mutable_view().permute(1, 0)
@@ -677,7 +676,7 @@ def path_ops(phase, ev, args):
     def scat():
         zt[[]] = y
     yh = y.to_numpy() if O else None
-    entry("transpose_scatter", "k_copy_tiled_v (LDS 128x128 tiles, 16-byte lanes)", scat, 8 * nn,
+    entry("transpose_scatter", "k_copy_tiled (LDS tiles, 16-byte lanes)", scat, 8 * nn,
           lambda: _cpu_leg(lambda: O.view_scatter(xh.copy(), [("permute", [1, 0])], r, yh[:rows]),
                            8 * rows * n, "view_scatter through z.mutable_view.permute(1, 0)",
                            f"its first {rows} rows"))
