@@ -268,8 +268,8 @@ bool cut(const Tile &t, int64_t ny, int64_t nx, int64_t k, Cut *c) {
 // (Float64) and 4% (Float32) of the best tile on average.  The fit is of tiles
 // dealt to the XCDs in turn: a grid beyond the 256 MB MALL streamed at 4.7 TB/s
 // at most, a little less in large tiles (8192^2, one step: Float64 219 us in
-// tiles of 4096 cells, 245 in 24576); in eighths it reaches 5.4 TB/s, which
-// leaves the order of the tiles as it is.
+// tiles of 4096 cells, 245 in 24576).  In eighths it reaches 5.4 TB/s; the
+// constants were not fitted again.
 template <typename T>
 double pass_us(const Tile &t, int64_t ny, int64_t nx, int64_t k, const Cut &c) {
   constexpr bool f64 = sizeof(T) == 8;
