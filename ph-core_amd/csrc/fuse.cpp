@@ -3591,6 +3591,7 @@ static int reduce_impl(const ph_prog *prog, int32_t n_in, const void *const *ins
     row_mode = true;
   }
   // whether dims [lo, hi) of v are one run of equal stride; its extent and stride
+  // (axes of one element are passed over: their strides address nothing)
   auto run_of = [](const ph_affine &v, int lo, int hi, int64_t *n, int64_t *st) {
     *n = 1;
     *st = 0;
@@ -3624,13 +3625,9 @@ static int reduce_impl(const ph_prog *prog, int32_t n_in, const void *const *ins
     if (!need_copy) {
       // can the needed 2-D split be expressed by strides?
       int split = (keep_axis == -1 || col_mode) ? rank - 1 : 1;  // dims [0,split) -> rows
-      for (int i = 0; i + 1 < split; ++i)
-        if (d.view.shape[i + 1] != 1 && d.view.stride[i] != d.view.stride[i + 1] * d.view.shape[i + 1])
-          need_copy = true;
-      bool one_run = true;
-      for (int i = split; i + 1 < rank; ++i)
-        if (d.view.shape[i + 1] != 1 && d.view.stride[i] != d.view.stride[i + 1] * d.view.shape[i + 1]) one_run = false;
       int64_t n, st;
+      if (!run_of(d.view, 0, split, &n, &st)) need_copy = true;
+      const bool one_run = run_of(d.view, split, rank, &n, &st);
       const bool parts = middle && run_of(d.view, 1, 1 + keep_axis, &n, &st) && run_of(d.view, 1 + keep_axis, rank, &n, &st);
       if (!one_run && parts) two_part = true;
       else if (!one_run) need_copy = true;
