@@ -101,10 +101,14 @@ int clear_i32(int *p, int n);
       return ph::set_error(PH_E_NOINIT, "ph_init has not been called");     \
   } while (0)
 
+// (The error is also taken off the runtime's own record, where the next
+// check_launch would find it.)
 #define PH_HIP(call)                                                         \
   do {                                                                       \
     hipError_t e_ = (call);                                                  \
-    if (e_ != hipSuccess)                                                    \
+    if (e_ != hipSuccess) {                                                  \
+      (void)hipGetLastError();                                               \
       return ph::set_error(PH_E_HIP, "%s failed: %s", #call,                 \
                            hipGetErrorString(e_));                           \
+    }                                                                        \
   } while (0)

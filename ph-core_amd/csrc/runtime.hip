@@ -3,6 +3,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -20,6 +21,7 @@ struct Scratch {
   size_t bytes = 0;
 };
 Scratch g_scratch[12];
+std::map<uintptr_t, size_t> g_buffers;  // ph_alloc's, by address
 long g_launches = 0;
 long g_fail_after = -2;  // -2: not read yet, -1: disabled
 }  // namespace
@@ -61,9 +63,18 @@ int scratch(size_t bytes, void **out, int slot) {
   return PH_OK;
 }
 
+// The buffer of ph_alloc that holds address p, or the end.
+static std::map<uintptr_t, size_t>::const_iterator buffer_of(const void *p) {
+  auto it = g_buffers.upper_bound((uintptr_t)p);
+  if (it == g_buffers.begin()) return g_buffers.end();
+  --it;
+  return (uintptr_t)p - it->first < it->second ? it : g_buffers.end();
+}
+
 // Copies small results to the host through a page of coherent host memory that
 // a kernel writes: the runtime's own copy to pageable memory stages them as
-// well, at several times the overhead.
+// well, at several times the overhead.  The kernel reads src as it is, so
+// callers pass library memory only, of at least `bytes`.
 static __global__ void k_to_host(char *__restrict__ dst, const char *__restrict__ src, unsigned bytes) {
   const unsigned t = blockIdx.x * blockDim.x + threadIdx.x, n = gridDim.x * blockDim.x;
   const bool words = ((uintptr_t)src & 7) == 0;
@@ -270,6 +281,7 @@ int ph_alloc(void **ptr, size_t bytes) {
     (void)hipGetLastError();
     return ph::set_error(PH_E_OOM, "hipMalloc of %zu bytes failed", bytes);
   }
+  ph::g_buffers[(uintptr_t)*ptr] = bytes;
   return PH_OK;
 }
 
@@ -279,6 +291,7 @@ int ph_free(void *ptr) {
   if (!ptr) return PH_OK;
   PH_HIP(hipStreamSynchronize(ph::g_stream));
   PH_HIP(hipFree(ptr));
+  ph::g_buffers.erase((uintptr_t)ptr);
   return PH_OK;
 }
 
@@ -296,7 +309,24 @@ int ph_d2h(void *dst, const void *src, size_t bytes) {
   PH_GUARD();
   PH_REQUIRE_INIT();
   if (bytes == 0) return PH_OK;
-  return ph::fetch(dst, src, bytes);
+  // A kernel reads the source of a small copy, and the host writes its
+  // destination, so that route is for the library's own buffers and for host
+  // memory.  Anything else (a null or foreign address, host memory as the
+  // source) goes to the runtime's copy, which checks it and reports an error.
+  const auto b = ph::buffer_of(src);
+  if (b != ph::g_buffers.end()) {
+    if (bytes > b->second - ((uintptr_t)src - b->first))
+      return ph::set_error(PH_E_HIP, "ph_d2h: %zu bytes from byte %zu of a buffer of %zu", bytes,
+                           (size_t)((uintptr_t)src - b->first), b->second);
+    hipPointerAttribute_t at;
+    const bool known = dst && hipPointerGetAttributes(&at, dst) == hipSuccess;
+    if (!known) (void)hipGetLastError();  // (ordinary host memory, to some runtimes an error)
+    if (dst && (!known || at.type == hipMemoryTypeUnregistered || at.type == hipMemoryTypeHost))
+      return ph::fetch(dst, src, bytes);
+  }
+  PH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ph::g_stream));
+  PH_HIP(hipStreamSynchronize(ph::g_stream));
+  return PH_OK;
 }
 
 int ph_d2d(void *dst, const void *src, size_t bytes) {
