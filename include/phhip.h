@@ -559,7 +559,9 @@ long ph_jit_compiles(void);
 /* Number of device operations issued so far: each kernel launch, or each
  * fixed sequence of launches one entry point issues as a unit (a reduction's
  * tile and finish kernels, a batch pass), counts once.  PH_HIP_FAIL_AFTER=n
- * (read at the first launch) refuses every operation after the first n. */
+ * (read at the first launch) refuses every operation after the first n, and
+ * PH_HIP_FAIL_AFTER=n+k the launches of operation n+1 after its first k (of a
+ * reduction; nothing else is refused then). */
 long ph_launch_count(void);
 
 #ifdef __cplusplus

@@ -73,8 +73,12 @@ void collapse(const ph_view_desc *const *descs, int nops, Layout *out);
 
 // Counts launches; PH_HIP_FAIL_AFTER=n makes launch n+1 (and later) fail with
 // PH_E_HIP before it is issued, so host code can exercise its device-error
-// handling without a faulting kernel.
+// handling without a faulting kernel.  PH_HIP_FAIL_AFTER=n+k (k >= 1) refuses
+// the launches after the first k of operation n+1 instead, and nothing later:
+// launch_step stands before each further launch of an operation whose failure
+// has to leave the library in order (a reduction's folds and finish).
 int launch_gate(const char *what);
+int launch_step(const char *what);
 long launch_count();
 
 // Generates and compiles (no launch) the general batch kernels for `prog`

@@ -739,25 +739,28 @@ int64_t grid_for(int64_t blocks) {
 // a copy back after it: only the wait for the stream, which the caller's
 // exception requires.  (Two checked operators on a 32 x 48 Int32 array took 58
 // us with a clear, a copy and a wait each.)  Guard and host words are zero
-// between calls: read_flags clears what a call raised, under the ABI lock.  A
-// call without flags_out raises into a block of its own that is never read.
+// between calls: read_flags clears what a call raised, under the ABI lock, and
+// get_flags_buffer does where a call failed on its way there.  A call without
+// flags_out raises into a block of its own that is never read.
 struct FlagBlock {
   int *dev = nullptr;   // guard, ticket, address of the host words
   int *host = nullptr;  // one word per bit
+  bool unread = false;  // a call took the block and has not read its flags
 };
 constexpr int kFlagBits = 4;   // the PH_FLAG_* bits, and kMaybeOverflow
 constexpr int kMaybeOverflow = 8;
 
-int *g_flag_host = nullptr;  // the host words of the block that is read
+FlagBlock g_flags[2];  // read, never read
 
+// The device words of a call's flags; `wanted`: the call will read them.
 int get_flags_buffer(int **dflags, bool wanted) {
-  static FlagBlock blocks[2];  // read, never read
-  FlagBlock &b = blocks[wanted ? 0 : 1];
+  FlagBlock &b = g_flags[wanted ? 0 : 1];
   if (!b.dev) {
     int *host = nullptr, *dev = nullptr;
     PH_HIP(hipHostMalloc((void **)&host, 64, hipHostMallocCoherent));
     std::memset(host, 0, 64);
     if (hipMalloc((void **)&dev, 64) != hipSuccess) {
+      (void)hipGetLastError();
       (void)hipHostFree(host);
       return ph::set_error(PH_E_OOM, "flag words");
     }
@@ -768,23 +771,34 @@ int get_flags_buffer(int **dflags, bool wanted) {
     b.dev = dev;
     b.host = host;
   }
-  if (wanted) g_flag_host = b.host;
+  if (wanted && b.unread) {
+    // an earlier call failed after its kernels were launched: what they raised
+    // is not this call's
+    PH_HIP(hipStreamSynchronize(ph::stream()));
+    std::memset(b.host, 0, kFlagBits * sizeof(int));
+    const int rc = ph::clear_i32(b.dev, 1);
+    if (rc) return rc;
+  }
+  b.unread = wanted;
   *dflags = b.dev;
   return PH_OK;
 }
 
-int read_flags(int *dflags, bool may_flag, int32_t *flags_out) {
-  if (!flags_out) return PH_OK;
-  *flags_out = 0;
-  if (!may_flag) return PH_OK;
+// The flags of a call that took its block as `wanted`.
+int read_flags(bool wanted, int32_t *flags_out) {
+  if (flags_out) *flags_out = 0;
+  if (!wanted) return PH_OK;
+  FlagBlock &b = g_flags[0];
   PH_HIP(hipStreamSynchronize(ph::stream()));
-  volatile int *h = g_flag_host;
+  volatile int *h = b.host;
   for (int k = 0; k < kFlagBits; ++k)
     if (h[k]) {
       *flags_out |= 1 << k;
       h[k] = 0;
     }
-  return *flags_out ? ph::clear_i32(dflags, 1) : PH_OK;
+  const int rc = *flags_out ? ph::clear_i32(b.dev, 1) : PH_OK;
+  if (!rc) b.unread = false;
+  return rc;
 }
 
 // Compiled fused kernels, keyed by everything their source depends on (the
@@ -1835,7 +1849,8 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
     }
     fused_cache()[key] = FusedKernels{{ktile, kfin, kfold}, 0};
   }
-  const bool may_flag = prog_may_flag(prog) || (std::string(P.state) == "SI" && (full_sum || row_sum || col_sum));
+  const bool want_flags =
+      flags_out && (prog_may_flag(prog) || (std::string(P.state) == "SI" && (full_sum || row_sum || col_sum)));
   // scratch: rowpart [ntc][rows], colpart [ntr][cols], rowfinal [row blocks of 256] (sized [rows]),
   // the first pre-fold levels [ntc / 64][rows] and [ntr / 64][cols]
   const size_t rowpart_b = P.do_rows ? (size_t)(P.ntc * P.rows) * P.state_bytes : 0;
@@ -1850,7 +1865,7 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
                    &base, 2);
   if (rc) return rc;
   int *dflags;
-  rc = get_flags_buffer(&dflags, flags_out != nullptr);
+  rc = get_flags_buffer(&dflags, want_flags);
   if (rc) return rc;
   RedArgs A;
   std::memset(&A, 0, sizeof(A));
@@ -1895,27 +1910,30 @@ int run_reduce2d_once(const ph_prog *prog, int n_in, const void *const *ins, con
       F.rows = series;
       F.nin = n;
       F.nout = nout;
+      if (ph::launch_step("reduction pre-fold")) return nullptr;
       size_t fsz = sizeof(F);
       void *fcfg[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, &F, HIP_LAUNCH_PARAM_BUFFER_SIZE, &fsz, HIP_LAUNCH_PARAM_END};
       if (hipModuleLaunchKernel(kfold, (unsigned)((series * nout + 255) / 256), 1, 1, 256, 1, 1, 0, ph::stream(),
-                                nullptr, fcfg) != hipSuccess)
+                                nullptr, fcfg) != hipSuccess) {
+        ph::set_error(PH_E_HIP, "reduction pre-fold launch failed");
         return nullptr;
+      }
       n = nout;
       cur ^= 1;
     }
     return lv[cur];
   };
   char *spare = (char *)A.rowzero + al(rowzero_b);
-  if (fold_rows && !(A.rowpart = fold(A.rowpart, spare, P.rows, P.ntc, kRowFold)))
-    return ph::set_error(PH_E_HIP, "reduction pre-fold launch failed");
-  if (fold_cols && !(A.colpart = fold(A.colpart, spare + al(fold_b), P.cols, P.ntr, kColFold)))
-    return ph::set_error(PH_E_HIP, "reduction pre-fold launch failed");
+  if (fold_rows && !(A.rowpart = fold(A.rowpart, spare, P.rows, P.ntc, kRowFold))) return PH_E_HIP;
+  if (fold_cols && !(A.colpart = fold(A.colpart, spare + al(fold_b), P.cols, P.ntr, kColFold))) return PH_E_HIP;
   // finish: column blocks of 256 / parts columns, then row blocks of 256 rows
   const int64_t fc = 256 / P.parts;
   const int64_t nfin = (P.do_cols ? (P.cols + fc - 1) / fc : 0) + (P.do_rows ? (P.rows + 255) / 256 : 0);
+  rc = ph::launch_step("reduction finish");
+  if (rc) return rc;
   if (nfin > 0)
     PH_HIP(hipModuleLaunchKernel(kfin, (unsigned)nfin, 1, 1, 256, 1, 1, 0, ph::stream(), nullptr, cfg));
-  return read_flags(dflags, may_flag, flags_out);
+  return read_flags(want_flags, flags_out);
 }
 
 // Whether an output lies inside what the inputs' views read: the second run
@@ -2002,9 +2020,9 @@ int map_tiled(const ph_prog *prog, int n_in, const void *const *ins, const int *
     if (rc) return rc;
     fused_cache()[key] = FusedKernels{{fn, nullptr, nullptr}, nblocks};
   }
-  const bool may_flag = prog_may_flag(prog);
+  const bool want_flags = flags_out && prog_may_flag(prog);
   int *dflags;
-  int rc = get_flags_buffer(&dflags, flags_out != nullptr);
+  int rc = get_flags_buffer(&dflags, want_flags);
   if (rc) return rc;
   MapArgs A;
   std::memset(&A, 0, sizeof(A));
@@ -2020,7 +2038,7 @@ int map_tiled(const ph_prog *prog, int n_in, const void *const *ins, const int *
   rc = ph::launch_gate("map (tiled)");
   if (rc) return rc;
   PH_HIP(hipModuleLaunchKernel(fn, (unsigned)grid_for(nblocks), 1, 1, kBlock, 1, 1, 0, ph::stream(), nullptr, cfg));
-  return read_flags(dflags, may_flag, flags_out);
+  return read_flags(want_flags, flags_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -3472,9 +3490,9 @@ int ph_map(const ph_prog *prog, int32_t n_in, const void *const *ins, const ph_v
     if (rc) return rc;
     fused_cache()[key] = FusedKernels{{fn, nullptr, nullptr}, nblocks};
   }
-  const bool may_flag = prog_may_flag(prog);
+  const bool want_flags = flags_out && prog_may_flag(prog);
   int *dflags;
-  rc = get_flags_buffer(&dflags, flags_out != nullptr);
+  rc = get_flags_buffer(&dflags, want_flags);
   if (rc) return rc;
   MapArgs A;
   std::memset(&A, 0, sizeof(A));
@@ -3492,7 +3510,7 @@ int ph_map(const ph_prog *prog, int32_t n_in, const void *const *ins, const ph_v
   if (rc) return rc;
   PH_HIP(hipModuleLaunchKernel(fn, (unsigned)grid_for(nblocks), 1, 1, kBlock, 1, 1, 0, ph::stream(),
                                nullptr, cfg));
-  return read_flags(dflags, may_flag, flags_out);
+  return read_flags(want_flags, flags_out);
 }
 
 // `colex`: the caller's view is the transpose of in_descs, so its

@@ -24,6 +24,8 @@ Scratch g_scratch[12];
 std::map<uintptr_t, size_t> g_buffers;  // ph_alloc's, by address
 long g_launches = 0;
 long g_fail_after = -2;  // -2: not read yet, -1: disabled
+long g_fail_step = 0;    // launches of that operation that still run (0: none, and none of the later ones)
+long g_step = 0;         // launches of the current operation
 }  // namespace
 
 int set_error(int code, const char *fmt, ...) {
@@ -211,10 +213,20 @@ int launch_gate(const char *what) {
   if (g_fail_after == -2) {
     const char *e = std::getenv("PH_HIP_FAIL_AFTER");
     g_fail_after = e ? std::atol(e) : -1;
+    const char *plus = e ? std::strchr(e, '+') : nullptr;
+    g_fail_step = plus ? std::atol(plus + 1) : 0;
   }
-  if (g_fail_after >= 0 && g_launches >= g_fail_after)
+  if (g_fail_after >= 0 && g_fail_step == 0 && g_launches >= g_fail_after)
     return set_error(PH_E_HIP, "%s: launch refused by PH_HIP_FAIL_AFTER=%ld", what, g_fail_after);
   ++g_launches;
+  g_step = 1;
+  return PH_OK;
+}
+
+int launch_step(const char *what) {
+  ++g_step;
+  if (g_fail_step > 0 && g_launches == g_fail_after + 1 && g_step > g_fail_step)
+    return set_error(PH_E_HIP, "%s: launch refused by PH_HIP_FAIL_AFTER=%ld+%ld", what, g_fail_after, g_fail_step);
   return PH_OK;
 }
 
