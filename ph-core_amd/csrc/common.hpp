@@ -89,6 +89,9 @@ int gbatch_compile_check(const ph_prog *prog, int x_dtype);
 // Looks up, for `device` (current), the device address of the fixed array
 // ph_heat2d_noalloc keeps its partial sums in (heat.hip).
 int heat_noalloc_setup(int device);
+
+// Sets up the words that maps and reductions raise their flags in (fuse.cpp).
+int flags_setup();
 int check_launch(const char *what);
 
 // Zeroes n int32 words on the library stream with a kernel (a memset node

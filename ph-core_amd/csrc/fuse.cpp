@@ -750,27 +750,11 @@ struct FlagBlock {
 constexpr int kFlagBits = 4;   // the PH_FLAG_* bits, and kMaybeOverflow
 constexpr int kMaybeOverflow = 8;
 
-FlagBlock g_flags[2];  // read, never read
+FlagBlock g_flags[2];  // read, never read (set up by ph_init: a first call may be captured)
 
 // The device words of a call's flags; `wanted`: the call will read them.
 int get_flags_buffer(int **dflags, bool wanted) {
   FlagBlock &b = g_flags[wanted ? 0 : 1];
-  if (!b.dev) {
-    int *host = nullptr, *dev = nullptr;
-    PH_HIP(hipHostMalloc((void **)&host, 64, hipHostMallocCoherent));
-    std::memset(host, 0, 64);
-    if (hipMalloc((void **)&dev, 64) != hipSuccess) {
-      (void)hipGetLastError();
-      (void)hipHostFree(host);
-      return ph::set_error(PH_E_OOM, "flag words");
-    }
-    int init[16] = {0};
-    std::memcpy(init + 2, &host, sizeof(host));
-    PH_HIP(hipMemcpyAsync(dev, init, 64, hipMemcpyHostToDevice, ph::stream()));
-    PH_HIP(hipStreamSynchronize(ph::stream()));
-    b.dev = dev;
-    b.host = host;
-  }
   if (wanted && b.unread) {
     // an earlier call failed after its kernels were launched: what they raised
     // is not this call's
@@ -3095,6 +3079,29 @@ int hazard_inputs(int n_in, const void *const *ins, const ph_view_desc *in_descs
 }  // namespace
 
 namespace ph {
+
+int flags_setup() {
+  for (FlagBlock &b : g_flags) {
+    if (b.dev) continue;
+    int *host = nullptr, *dev = nullptr;
+    PH_HIP(hipHostMalloc((void **)&host, 64, hipHostMallocCoherent));
+    std::memset(host, 0, 64);
+    int init[16] = {0};
+    std::memcpy(init + 2, &host, sizeof(host));
+    hipError_t e = hipMalloc((void **)&dev, 64);
+    if (e == hipSuccess) e = hipMemcpyAsync(dev, init, 64, hipMemcpyHostToDevice, stream());
+    if (e == hipSuccess) e = hipStreamSynchronize(stream());
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      if (dev) (void)hipFree(dev);
+      (void)hipHostFree(host);
+      return set_error(e == hipErrorOutOfMemory ? PH_E_OOM : PH_E_HIP, "flag words: %s", hipGetErrorString(e));
+    }
+    b.dev = dev;
+    b.host = host;
+  }
+  return PH_OK;
+}
 
 int ordered_copy(void *dst, const ph_view_desc *dd, const void *src, const ph_view_desc *sd, bool *done) {
   *done = false;
