@@ -1955,11 +1955,12 @@ int run_reduce2d(const ph_prog *prog, int n_in, const void *const *ins, const in
   }
   int rc = run_reduce2d_once(prog, n_in, ins, in_dt, V, acc, full_sum, full_max, row_sum, row_max, col_sum, col_max,
                              flags_out, colex, bounds);
-  if (rc || !flags_out || !(*flags_out & kMaybeOverflow)) return rc;
-  if (*flags_out & PH_FLAG_OVERFLOW) {
-    *flags_out &= ~kMaybeOverflow;
-    return rc;
-  }
+  // (kMaybeOverflow is between the two runs: the caller never sees it, also not
+  // where one of them fails)
+  const bool maybe = flags_out && (*flags_out & kMaybeOverflow);
+  if (maybe) *flags_out &= ~kMaybeOverflow;
+  if (rc || !maybe || (*flags_out & PH_FLAG_OVERFLOW)) return rc;
+  *flags_out = 0;
   return run_reduce2d_once(prog, n_in, ins, in_dt, V, acc, full_sum, full_max, row_sum, row_max, col_sum, col_max,
                            flags_out, colex, false);
 }

@@ -51,3 +51,30 @@ def test_flags_of_a_failed_reduction_are_dropped(shape, what):
         print("clean")
     """, "0+1")
     assert "clean" in out
+
+
+def test_second_run_of_a_bounded_sum_refused():
+    """Int32 values whose bounds leave Int32 and whose totals do not: the exact
+    run that would decide is refused, and the flags hold none of the first's."""
+    out = _child("""
+        import ctypes as C
+        import os
+        import numpy as np
+        import phase
+        from test_gpu_alias_deep import _desc
+
+        class Prog(C.Structure):  # r0 = input 0
+            _fields_ = [(n, C.c_int32) for n in ("n_insn", "n_in", "out_reg", "out_dtype")] + [("insn", C.c_int64 * 96)]
+
+        phase.init(0)
+        lib = C.CDLL(os.path.join(phase.LIB_DIR, "libphhip.so"))
+        top = 2**31 - 1
+        x = phase.NArray.from_numpy(np.array([top, -top] * 50, np.int32))
+        s = phase.NArray.from_numpy(np.zeros(1))
+        d, p = _desc(0, 100, [100]), Prog(1, 1, 0, 0)
+        ins, fl = (C.c_void_p * 1)(x.device_ptr), C.c_int32(77)
+        rc = lib.ph_reduce(C.byref(p), 1, ins, C.byref(d), -1, 1, 0, C.c_void_p(s.device_ptr), None, C.byref(fl))
+        assert rc == -10 and fl.value == 0, (rc, fl.value)
+        print("refused")
+    """, "1")
+    assert "refused" in out
