@@ -1203,14 +1203,21 @@ std::string red_tile_float(const ph_prog *p, int n_in, const int *in_dt, const i
   // the previous group's data)
   auto loads = [&](const std::string &b, const std::string &g) {
     std::string o;
-    // (where the rows are checked, by a 32-bit minimum: of a 64-bit compare and
-    // select the compiler sank a row's select past the compare of its branch
-    // and read the wrong row, with columns in two parts)
-    if (chk_rows || P.cols2)
-      o += "#pragma unroll\n    for (int k = 0; k < 8; ++k) {\n      const int rk = (int)(" + g +
-           " - r0) + k;\n      const i64 r = r0 + (rk < nr ? rk : nr - 1);\n";
+    // (by 32-bit selects: of a 64-bit compare and select a row, the compiler
+    // sank one row's select past the compare of a branch, and row 1 of a tile
+    // read the tile's last row.  A whole tile has a multiple of 16 rows, so one
+    // select serves a group: past the end a tall tile reads its last eight rows
+    // again, a low one its last row eight times.  Float32 16384^2 (512 rows a tile)
+    // 183.4 us, Float64 4096^2 (32 rows) 29.8, as with a 64-bit select a row; the
+    // other way round 183.6 and 31.2, and with a 32-bit select a row 186.2 and 29.9.)
+    const std::string gk = "    const int gk = (int)(" + g + " - r0);\n", rows8 = "#pragma unroll\n    for (int k = 0; k < 8; ++k) {\n";
+    if (chk_rows)
+      o += gk + rows8 + "      const i64 r = r0 + (gk + k < nr ? gk + k : nr - 1);\n";
+    else if (P.tr >= 128)
+      o += gk + fmt("    const i64 gr = r0 + (gk < %d ? gk : %d);\n", P.tr - 8, P.tr - 8) + rows8 + "      const i64 r = gr + k;\n";
     else
-      o += "#pragma unroll\n    for (int k = 0; k < 8; ++k) {\n      const i64 r = (" + g + " + k < r1) ? " + g + " + k : r1 - 1;\n";
+      o += gk + fmt("    const int gs = gk < %d ? 1 : 0;\n    const i64 gr = r0 + (gs ? gk : %d);\n", P.tr, P.tr - 1) + rows8 +
+           "      const i64 r = gr + k * gs;\n";
     o += "      {\n";
     for (int j = 0; j < n_in; ++j) {
       o += fmt("        const %s *rp%d = (const %s *)A.in[%d] + (A.in_off[%d] + r * %s);\n", stype(in_dt[j]), j,

@@ -63,3 +63,18 @@ def test_middle_axis_order(ph):
     z[0, 1, 5], z[2, 1, 1] = 0.0, -0.0
     m = ph.NArray.from_numpy(z).slices_max(1)
     assert np.signbit(m[0]) and not np.signbit(m[1]) and m == [0.0, 0.0]
+
+
+@pytest.mark.parametrize("dt", [np.float64, np.float32, np.int32])
+def test_every_row_of_a_tile_is_its_own(ph, dt):
+    """Every element of a slice holds the slice's number, so a row of a tile
+    that is read in another's place shows: tiles with and without missing
+    rows and columns, the kept axis in the middle and in front."""
+    for shape, k in [((4, 16, 512), 1), ((4, 33, 512), 1), ((8, 129, 515), 1), ((96, 1000, 515), 1), ((2, 96, 2048), 1),
+                     ((33, 1030), 0), ((160, 1024), 0)]:
+        j = np.arange(shape[k])
+        h = np.broadcast_to(j.reshape([-1 if a == k else 1 for a in range(len(shape))]), shape)
+        x = ph.NArray.from_numpy(np.ascontiguousarray(h).astype(dt))
+        n = h.size // shape[k]
+        assert x.slices_max(k) == [float(v) for v in j], (shape, k)
+        assert x.slices_sum(k) == [float(v) for v in j * n], (shape, k)
