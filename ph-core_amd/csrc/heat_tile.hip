@@ -53,8 +53,11 @@ struct TileArgs {
 
 // kMask: the grid is narrower or lower than a tile, so the cells of the tile
 // beyond the grid are held at zero after every step.
+// Eight wavefronts to a SIMD are asked for in whole tiles of 16 wavefronts: the
+// separate form of 128 x 256 Float32 took 65 registers, one too many for two
+// workgroups on a CU (8192^2, 20 steps a pass: 477 us, and 340 with 64).
 template <typename T, int V, int R, int W, bool kFused, bool kMask>
-__global__ __launch_bounds__(64 * W) void k_heat_tile(const T *u, T *out, TileArgs a, T r) {
+__global__ __launch_bounds__(64 * W, W == 16 && !kMask ? 8 : 0) void k_heat_tile(const T *u, T *out, TileArgs a, T r) {
   constexpr int TX = 64 * V, TY = W * R;
   typedef T Row __attribute__((ext_vector_type(V)));
   struct __attribute__((packed, aligned(sizeof(T)))) RowU {
