@@ -204,11 +204,6 @@ int fused_safe(const T *u, int64_t n, T r, bool *safe, int64_t *steps_ok) {
   return PH_OK;
 }
 
-// Most workgroups of a pass that leave the field's energy as one partial sum
-// each (two sums of a pass fill the fixed array of ph_heat2d_noalloc).  Passes
-// of more (grids of more than about 10^8 cells) sum the field in a pass of its own.
-constexpr int64_t kEnergyGroups = 8192;
-
 // part_buf / part_cap: a fixed buffer for the energy partials (the
 // allocation-free entry point); allow_fused: the fused first operation may
 // be used (it needs one read-back of max|u|).
@@ -219,6 +214,8 @@ int heat_run(T *u, T *tmp, int64_t ny, int64_t nx, double r, int64_t steps, int6
   // length by the tile and pass plan; PH_HEAT_K caps the steps of a pass.
   int64_t kmax = INT32_MAX;
   if (const char *e = std::getenv("PH_HEAT_K")) kmax = std::max<int64_t>(1, std::atol(e));
+  int only = -1;
+  if (const char *e = std::getenv("PH_HEAT_TILE")) only = std::atoi(e);  // tuning override: one tile of heat_tile.hip
   const T rr = (T)r;
   const bool sums = energy && every > 0;
   T *cur = u;
@@ -226,6 +223,8 @@ int heat_run(T *u, T *tmp, int64_t ny, int64_t nx, double r, int64_t steps, int6
   if (sums && steps == 0) return fp64_sum<T, T, 1>(u, u, ny * nx, energy, part_buf, part_cap);
   // one grid copy, which an odd number of passes needs at the end
   const double copy_us = 4.0 + 2.0 * sizeof(T) * (double)ny * (double)nx / 5e6;
+  // and the field's energy in a pass of its own
+  const double sum_us = sums ? 6.0 + sizeof(T) * (double)ny * (double)nx / 3.1e6 : 0.0;
   bool fused = false, try_fused = false;
   int64_t fused_until = 0;
   Pass p{-1, 0, 0, false, 0.0};
@@ -236,7 +235,7 @@ int heat_run(T *u, T *tmp, int64_t ny, int64_t nx, double r, int64_t steps, int6
     const int64_t span = until - t;
     if (span != planned || until == steps) {
       // the last passes should leave the field in u
-      p = plan<T>(ny, nx, span, kmax, until == steps ? (cur == u ? 0 : 1) : -1, copy_us);
+      p = plan<T>(ny, nx, span, kmax, until == steps ? (cur == u ? 0 : 1) : -1, copy_us, sum_us, only);
       planned = span;
       if (p.tile < 0) return ph::set_error(PH_E_UNSUPPORTED, "heat grid %lld x %lld", (long long)ny, (long long)nx);
     }

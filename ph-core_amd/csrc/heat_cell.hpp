@@ -74,11 +74,18 @@ struct Pass {
   bool one;         // one tile covers the grid: in and out may be the same buffer
   double us;        // predicted time of all the passes
 };
+// Most workgroups of a pass that leave the field's energy as one partial sum
+// each (two sums of a pass fill the fixed array of ph_heat2d_noalloc).  Passes
+// of more sum the field in a pass of its own.
+constexpr int64_t kEnergyGroups = 8192;
 // The tile, and the number of passes, for `span` steps (span >= 1) of a
 // ny x nx grid with at most kmax steps per pass.  parity 0 or 1: a number of
 // passes of the other parity costs one copy of the grid (copy_us) more.
+// Passes of more than kEnergyGroups groups cost sum_us more (the energy at the
+// span's end takes a pass of its own).  only >= 0: that tile alone, where it can take the grid.
 template <typename T>
-Pass plan(int64_t ny, int64_t nx, int64_t span, int64_t kmax, int parity, double copy_us);
+Pass plan(int64_t ny, int64_t nx, int64_t span, int64_t kmax, int parity, double copy_us, double sum_us,
+          int only);
 // One pass of `steps` steps, cur -> nxt.  part0 / part1, when given, receive
 // one compensated sum per workgroup of the field before / after the pass
 // (*groups of them, at most p.groups); a lone workgroup writes the sum itself,

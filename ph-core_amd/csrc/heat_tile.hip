@@ -23,9 +23,10 @@
 // additions) and 8.1 at Float64 (six, and two shifts of two words each per
 // pair of cells).  At 8192^2 that keeps the vector ALUs 96% busy at Float32;
 // the rest is the overlap (a third of the cells at 16 steps and 128 x 256).
-// Time per step, the sweep's and this kernel's, over runs of 100 steps (passes
-// of at most two steps may lose: Float32 8192^2 59 -> 62 us, 5000 x 7000 31 -> 35):
-//   8192^2     Float32 18.5 -> 14.2 us, Float64 36 -> 27.4 us
+// Time per step, the sweep's and this kernel's, over runs of 100 steps (and in
+// passes of one step and of two: 8192^2 Float32 116 -> 102 and 59 -> 51 us, Float64
+// 233 -> 196 and 119 -> 97):
+//   8192^2     Float32 18.6 -> 13.9 us, Float64 36 -> 27.8 us
 //   2048^2     Float32 3.9 -> 1.58, Float64 5.6 -> 3.0 us
 //   1024^2     Float32 3.6 -> 0.89, Float64 3.9 -> 1.27 us
 //   750 x 1111 Float32 6.1 -> 0.88, Float64 5.8 -> 1.18 us
@@ -65,8 +66,8 @@ __global__ __launch_bounds__(64 * W, W == 16 && !kMask ? 8 : 0) void k_heat_tile
   };
   __shared__ D2 esh[W];
   // [buffer][wavefront + 1][first, last row]; the rows beyond the first and
-  // last wavefront stay zero
-  __shared__ T sh[2][W + 2][2][TX];
+  // last wavefront stay zero (a lone wavefront exchanges none)
+  __shared__ T sh[2][W + 2][2][W > 1 ? TX : 1];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   // Each XCD (workgroups are dealt to the eight in turn) takes an eighth of the
@@ -102,10 +103,16 @@ __global__ __launch_bounds__(64 * W, W == 16 && !kMask ? 8 : 0) void k_heat_tile
   for (int i = 0; i < R; ++i) {
     if constexpr (kMask) {
       const T *row = u + (i < nr ? y + i : a.ny - 1) * a.nx + xs;
+      if (nc == TX) {  // rows alone are missing
+        const RowU t = *(const RowU *)(row + (unsigned)lx);
 #pragma unroll
-      for (int v = 0; v < V; ++v) {
-        const T t = row[(unsigned)(colok[v] ? lx + v : 0)];
-        c[i][v] = (colok[v] && i < nr) ? t : T(0);
+        for (int v = 0; v < V; ++v) c[i][v] = i < nr ? t.v[v] : T(0);
+      } else {
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+          const T t = row[(unsigned)(colok[v] ? lx + v : 0)];
+          c[i][v] = (colok[v] && i < nr) ? t : T(0);
+        }
       }
     } else {
       const T *row = u + (y + i) * a.nx + xs;
@@ -180,15 +187,21 @@ __global__ __launch_bounds__(64 * W, W == 16 && !kMask ? 8 : 0) void k_heat_tile
     __syncthreads();
   };
   if (a.part0) sum_to(a.part0);
-  for (int i = threadIdx.x; i < 2 * TX; i += 64 * W) sh[i / TX][0][1][i % TX] = sh[i / TX][W + 1][0][i % TX] = T(0);
+  if constexpr (W > 1)
+    for (int i = threadIdx.x; i < 2 * TX; i += 64 * W) sh[i / TX][0][1][i % TX] = sh[i / TX][W + 1][0][i % TX] = T(0);
   for (int s = 0; s < a.steps; ++s) {
-    T(*b)[2][TX] = sh[s & 1];
-    put(c[0], b[wave + 1][0]);
-    put(c[R - 1], b[wave + 1][1]);
+    auto *b = sh[s & 1];
     T second[V], nn[V], nx4[V], up[V], dn[V];
+    if constexpr (W > 1) {
+      put(c[0], b[wave + 1][0]);
+      put(c[R - 1], b[wave + 1][1]);
+    } else {  // a lone wavefront holds all rows: beyond them is the boundary
 #pragma unroll
-    for (int v = 0; v < V; ++v) second[v] = c[1][v];
-    north(c[0], 1, nn);
+      for (int v = 0; v < V; ++v) up[v] = dn[v] = T(0);
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) second[v] = R > 1 ? c[R > 1][v] : T(0);
+    if constexpr (R > 1) north(c[0], 1, nn);
     // Rows are updated in place, top down: a row's north - 4 centre is taken
     // before the row above it changes.  Half of the inner rows run before the
     // barrier, half while the neighbours' rows are read; the first row, whose
@@ -196,11 +209,12 @@ __global__ __launch_bounds__(64 * W, W == 16 && !kMask ? 8 : 0) void k_heat_tile
     constexpr int kHalf = (R - 2) / 2;
 #pragma unroll
     for (int i = 1; i < R; ++i) {
-      if (i == 1 + kHalf) {
-        __syncthreads();
-        get(b[wave][1], up);
-        get(b[wave + 2][0], dn);
-      }
+      if constexpr (W > 1)
+        if (i == 1 + kHalf) {
+          __syncthreads();
+          get(b[wave][1], up);
+          get(b[wave + 2][0], dn);
+        }
       if (i < R - 1) {
         north(c[i], i + 1, nx4);
         update(i, nn, c[i + 1]);
@@ -232,20 +246,32 @@ __global__ __launch_bounds__(64 * W, W == 16 && !kMask ? 8 : 0) void k_heat_tile
 }
 
 // The tiles, by dtype.  Measured over 24 grids from 33 x 47 to 8192^2 and 23
-// tiles: these eight leave the best of all 23 at most a few percent ahead
-// (the last ones serve the large grids, 64 x 32 the small ones, the narrow
-// rows of 64 x 48 and 64 x 64 a grid that fits one tile).
+// tiles: the first eight leave the best of all 23 at most a few percent ahead
+// (the last of them serve the large grids, 64 x 32 the small ones, the narrow
+// rows of 64 x 48 and 64 x 64 a grid that fits one tile).  The other nine are
+// for grids of few rows, where 32 rows and more would mostly hold cells beyond
+// the grid, or 64 columns mostly overlap: up to 16 rows one wavefront spans them,
+// without LDS or barrier, then two and four.  Per run of 100 steps (and of one), the
+// sweep, the first eight tiles alone, and all:
+//   1 x 10^7      Float32 2888 (68), 4119 (280),  127 (40) us, Float64 2650 (102), 6465 (321),  304 (59)
+//   4 x 4 10^6    Float32 1555 (54), 2033 (148),  290 (51) us, Float64 1711 (94),  3236 (195),  482 (85)
+//   16 x 10^6     Float32  949 (53),  660 (69),   342 (51) us, Float64 1211 (90),  1062 (97),   591 (85)
+//   50 x 5 10^5   Float32  805 (73), 1139 (80),   731 (80) us, Float64 1545 (181), 1448 (168), 1362 (172)
 struct Tile {
   int v, r, w;
 };
 template <typename T> struct Tiles;
 template <> struct Tiles<double> {
-  static constexpr Tile t[8] = {{1, 4, 8}, {1, 6, 8}, {1, 8, 8}, {2, 4, 8}, {2, 8, 8}, {2, 12, 8}, {2, 16, 8}, {2, 24, 8}};
+  [[maybe_unused]] static constexpr Tile t[17] = {{1, 4, 8},  {1, 6, 8},  {1, 8, 8}, {2, 4, 8}, {2, 8, 8},  {2, 12, 8},
+                                                  {2, 16, 8}, {2, 24, 8}, {4, 1, 1}, {4, 2, 1}, {4, 4, 1},  {4, 8, 1},
+                                                  {2, 16, 1}, {2, 12, 2}, {2, 16, 2}, {2, 12, 4}, {2, 16, 4}};
 };
 template <> struct Tiles<float> {
-  static constexpr Tile t[8] = {{1, 4, 8}, {1, 6, 8}, {1, 8, 8}, {2, 4, 8}, {2, 8, 16}, {2, 12, 8}, {2, 12, 16}, {2, 16, 16}};
+  [[maybe_unused]] static constexpr Tile t[17] = {{1, 4, 8},   {1, 6, 8},   {1, 8, 8}, {2, 4, 8}, {2, 8, 16}, {2, 12, 8},
+                                                  {2, 12, 16}, {2, 16, 16}, {4, 1, 1}, {4, 2, 1}, {4, 4, 1},  {4, 8, 1},
+                                                  {2, 16, 1},  {2, 12, 2},  {2, 16, 2}, {2, 12, 4}, {2, 16, 4}};
 };
-constexpr int kTiles = 8;
+constexpr int kTiles = 17;
 
 struct Cut {
   int64_t ux, uy, ntx, nty;
@@ -255,6 +281,7 @@ struct Cut {
 template <typename T>
 bool cut(const Tile &t, int64_t ny, int64_t nx, int64_t k, Cut *c) {
   const int64_t tx = 64 * t.v, ty = (int64_t)t.w * t.r;
+  if (t.w == 1 && ny > ty) return false;  // (a lone wavefront spans the rows)
   c->ux = nx > tx ? tx - 2 * k : nx;
   c->uy = ny > ty ? ty - 2 * k : ny;
   if ((nx > tx && c->ux < tx / 8) || (ny > ty && c->uy < ty / 8)) return false;
@@ -265,29 +292,47 @@ bool cut(const Tile &t, int64_t ny, int64_t nx, int64_t k, Cut *c) {
 
 // Predicted time (us) of one pass of k steps: the launch, then per step
 // either a workgroup's own latency (barrier and LDS exchange, and its work
-// alone on a CU) or, with several workgroups to a CU, the CU's throughput,
-// and the tiles' memory traffic.  The constants are a fit to 7000 timings
-// (17% rms over grids, tiles and steps); the choice it makes is within 3%
-// (Float64) and 4% (Float32) of the best tile on average.  The fit is of tiles
-// dealt to the XCDs in turn: a grid beyond the 256 MB MALL streamed at 4.7 TB/s
-// at most, a little less in large tiles (8192^2, one step: Float64 219 us in
-// tiles of 4096 cells, 245 in 24576).  In eighths it reaches 5.4 TB/s; the
-// constants were not fitted again.
+// alone on a CU, of which a lone wavefront has one SIMD of four) or, with
+// several workgroups to a CU, the CU's throughput, and the tiles' memory
+// traffic.  The constants of the tiles of eight wavefronts and more are a fit to
+// 7000 timings (17% rms over grids, tiles and steps), those of the smaller ones
+// minimise the time of the tiles chosen for 65 grids of 1 to 100 rows and up
+// to 10^6 columns and 20 others, 1 to 100 steps: on average within 3.7%
+// (Float32) and 2.7% (Float64) of the best tile and number of steps, and 16%
+// and 12% faster than with the first eight tiles alone.  A grid beyond the
+// 256 MB MALL is streamed: 5.6 TB/s (Float64) and 5.4 (Float32) at most, less in
+// tall tiles, in rows of 256 bytes and in few rows (8192^2, one step: Float64 195 us
+// in tiles of 4096 cells, 232 in 24576; Float32 101 us in 128 x 32, 114 in
+// 64 x 32, 121 in 128 x 24).
+struct Cost {
+  double launch, fixed, alone, shared;  // a step alone: fixed + alone * work; with others: shared * work
+};
+template <typename T>
+Cost cost(const Tile &t) {
+  if constexpr (sizeof(T) == 8)
+    return t.w == 1 ? Cost{2.3, 0.02, 1.4, 0.6} : t.w < 8 ? Cost{1.4, 0.7, 1.87, 1.07} : Cost{2.1, 0.129, 0.913, 0.805};
+  else
+    return t.w == 1 ? Cost{2.6, 0.1, 0.82, 0.69} : t.w < 8 ? Cost{2.3, 0.175, 0.76, 0.73} : Cost{t.w == 16 ? 0.7 : 2.5, 0.086, 0.831, 0.565};
+}
 template <typename T>
 double pass_us(const Tile &t, int64_t ny, int64_t nx, int64_t k, const Cut &c) {
   constexpr bool f64 = sizeof(T) == 8;
   const bool mask = nx < 64 * t.v || ny < (int64_t)t.w * t.r;
   const double insn = (f64 ? 6 * t.v + 4 : 5 * t.v) + (mask ? (f64 ? 2 : 1) * t.v : 0);
-  const double work = t.w / 4.0 * (t.r * insn + 8) * 4 / 2400;  // of a step, on a CU's four SIMDs
+  const double wave = (t.r * insn + 8) * 4 / 2400;  // of a step, of one wavefront
+  const double work = t.w / 4.0 * wave;             // on a CU's four SIMDs
   const double traffic = 64.0 * t.v * t.w * t.r * sizeof(T) * 2 * 256 / 5e6;
   const double g = (double)(c.ntx * c.nty) / 256;
   const double per_cu = g <= 1 ? 1 : (g < 6 ? std::ceil(g) : g + 0.4);
-  const double step = f64 ? std::max(0.129 + 0.913 * work, 0.805 * work * per_cu)
-                          : std::max(0.086 + 0.831 * work, 0.565 * work * per_cu);
-  const double launch = f64 ? 2.1 : (t.w == 16 ? 0.7 : 2.5);
-  const double us = launch + k * step + (f64 ? 0.486 : 0.685) * traffic * per_cu;
+  const Cost f = cost<T>(t);
+  const double step = std::max(f.fixed + f.alone * std::max(wave, work), f.shared * work * per_cu);
+  const double us = f.launch + k * step + (f64 ? (mask ? 0.38 : 0.486) : 0.685) * traffic * per_cu;
   const double bytes = 2.0 * sizeof(T) * (double)ny * (double)nx;
-  const double stream = bytes > 256e6 ? bytes / 4.7e6 * (1 + 0.004 * t.v * t.w * t.r / 16) : 0;
+  if (bytes <= 256e6) return us;
+  const double cells = t.v * t.w * t.r / 16.0;  // of a tile, in 1024
+  const bool few = t.w < 8 && c.nty > 1;
+  const double stream = f64 ? bytes / 5.65e6 * (1 + 0.009 * cells) * (t.v == 1 ? 1.02 : 1) * (few ? 1.08 : 1)
+                            : bytes / 5.4e6 * (1 + 0.005 * cells) * (t.v == 1 ? 1.09 : 1) * (few ? 1.2 : 1);
   return std::max(us, stream);
 }
 
@@ -318,24 +363,30 @@ namespace ph {
 namespace heat {
 
 template <typename T>
-Pass plan(int64_t ny, int64_t nx, int64_t span, int64_t kmax, int parity, double copy_us) {
+Pass plan(int64_t ny, int64_t nx, int64_t span, int64_t kmax, int parity, double copy_us, double sum_us, int only) {
   Pass best{-1, 0, 0, false, 0.0};
   for (int i = 0; i < kTiles; ++i) {
     const Tile &t = Tiles<T>::t[i];
+    if (only >= 0 ? i != only : t.w < 8 && ny > 2 * t.w * t.r) continue;  // (low tiles are for low grids)
     const bool one = nx <= 64 * t.v && ny <= (int64_t)t.w * t.r;
     // a launch holds the device for some milliseconds at most
     const int64_t kcap = std::min(kmax, one ? int64_t(4096) : int64_t(48));
+    int64_t seen = -1;
     for (int64_t k0 = one ? kcap : 1; k0 <= kcap; ++k0) {
       const int64_t passes = (span + k0 - 1) / k0;
       const int64_t k = (span + passes - 1) / passes;
+      if (passes == seen && k0 < span) continue;
+      seen = passes;
       Cut c;
       if (!cut<T>(t, ny, nx, k, &c)) break;  // more steps leave less of the tile
       double us = passes * pass_us<T>(t, ny, nx, k, c);
       if (!one && parity >= 0 && passes % 2 != parity) us += copy_us;
+      if (c.ntx * c.nty > kEnergyGroups) us += sum_us;
       if (best.tile < 0 || us < best.us) best = Pass{i, passes, c.ntx * c.nty, one, us};
       if (k0 >= span) break;
     }
   }
+  if (best.tile < 0 && only >= 0) return plan<T>(ny, nx, span, kmax, parity, copy_us, sum_us, -1);
   return best;
 }
 
@@ -363,12 +414,16 @@ int launch(const Pass &p, bool fused, const T *cur, T *nxt, int64_t ny, int64_t 
   return launch_index<T, 0>(p.tile, fused, mask, (unsigned)(c.ntx * c.nty), cur, nxt, a, r);
 }
 
-template Pass plan<float>(int64_t, int64_t, int64_t, int64_t, int, double);
-template Pass plan<double>(int64_t, int64_t, int64_t, int64_t, int, double);
-template int launch<float>(const Pass &, bool, const float *, float *, int64_t, int64_t, float, int64_t, D2 *, D2 *,
-                           int64_t *);
-template int launch<double>(const Pass &, bool, const double *, double *, int64_t, int64_t, double, int64_t, D2 *, D2 *,
-                            int64_t *);
+#define PH_HEAT_INSTANCE(T)                                                                \
+  template Pass plan<T>(int64_t, int64_t, int64_t, int64_t, int, double, double, int);      \
+  template int launch<T>(const Pass &, bool, const T *, T *, int64_t, int64_t, T, int64_t, D2 *, D2 *, int64_t *);
+// (the build compiles this file once per type, side by side)
+#ifdef PH_HEAT_T
+PH_HEAT_INSTANCE(PH_HEAT_T)
+#else
+PH_HEAT_INSTANCE(float)
+PH_HEAT_INSTANCE(double)
+#endif
 
 }  // namespace heat
 }  // namespace ph

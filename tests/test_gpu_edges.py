@@ -134,9 +134,8 @@ def test_beyond_2_31_elements(ph):
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_heat_edge_placed_sweeps(ph, dt):
-    """Grids whose rows allow whole-vector lanes: strips flush with the west
-    and east edges, the top band swept down and the bottom band up from the
-    grid's edge, two and eight steps per pass (17 = 8 + 8 + 1), bit-exact."""
+    """Grids of whole vectors and of a few columns more, tiles flush with every
+    edge, in runs of 2, 8 and 17 steps, bit-exact."""
     rng = np.random.default_rng(29)
     for ny, nx in [(40, 256), (300, 1000), (1000, 2048), (97, 260)]:
         for steps in (2, 8, 17):
@@ -205,17 +204,20 @@ def test_int32_division_by_constants(ph):
 
 @pytest.mark.parametrize("dt", [np.float64, np.float32])
 def test_heat_fused_first_operation(ph, dt):
-    """Runs of 32 steps or more compute uN - 4u as one fused multiply-add
-    once max|u| shows that 4u cannot overflow; the result must stay
-    bit-identical to the oracle's separate multiply and subtract, on grids
-    that take the clean, edge and masked sweeps."""
+    """Runs predicted at 300 us or more compute uN - 4u as one fused
+    multiply-add once max|u| shows that 4u cannot overflow; the result must
+    stay bit-identical to the oracle's separate multiply and subtract, on
+    grids of whole tiles and of less.  (The launch that asks for max|u| shows
+    that a run is long enough; shorter ones keep the separate operations.)"""
+    from test_gpu_heat_fused import launches
     rng = np.random.default_rng(71)
-    for ny, nx, steps in [(200, 249, 40), (300, 1000, 33), (65, 257, 35), (1000, 2048, 40), (7, 1, 32)]:
+    for ny, nx, steps, asked in [(200, 249, 800, 1), (300, 1000, 600, 1), (65, 257, 800, 1), (1000, 2048, 400, 1),
+                                 (7, 1, 1000, 1), (300, 1000, 33, 0), (7, 1, 32, 0)]:
         u0 = (rng.standard_normal((ny, nx)) * 1e3).astype(dt)
-        u = ph.NArray.from_numpy(u0)
-        e = ph.heat2d(u, 0.2, steps, every=8)
+        u, e, extra = launches(ph, u0, 0.2, steps, 8)
         ref, eref = O.heat2d(u0, 0.2, steps, every=8)
-        assert np.array_equal(u.to_numpy(), ref), (ny, nx, steps)
+        assert extra == asked, (ny, nx, steps)
+        assert np.array_equal(u, ref), (ny, nx, steps)
         assert np.allclose(e, eref, rtol=1e-13, atol=1e-300), (ny, nx, steps)
 
 
@@ -224,7 +226,8 @@ def test_heat_unfused_when_4u_may_overflow(ph, dt):
     """Grids whose 4u can overflow (values near the largest finite value),
     that hold an infinity or a NaN, or that step with r > 1/4 (values may
     grow) keep the separate multiply and subtract: bit-identical to the
-    oracle, infinities and NaN included."""
+    oracle, infinities and NaN included.  (34 steps keep it by their length;
+    test_gpu_heat_fused.py has runs that are asked.)"""
     big = np.finfo(dt).max
     rng = np.random.default_rng(73)
     cases = []
@@ -252,10 +255,8 @@ def test_heat_unfused_when_4u_may_overflow(ph, dt):
 
 
 def test_heat_fp32_twelve_step_passes(ph):
-    """Float32 runs of passes of twelve steps (three halo lanes): the fused
-    first operation (runs of 32 steps or more), the flush sweeps (rows in
-    whole vectors, a wavefront wide or more) and the masked sweep (ragged or
-    narrow grids), bit-exact against the oracle's Float32 formula (u + d*r
+    """Float32 runs of 36 to 48 steps on grids of whole tiles and on ragged and
+    narrow ones, bit-exact against the oracle's Float32 formula (u + d*r
     rounded once)."""
     rng = np.random.default_rng(79)
     for ny, nx in [(65, 257), (200, 249), (130, 5), (300, 1000), (1000, 2048), (97, 260), (40, 256)]:
