@@ -335,8 +335,11 @@ __global__ __launch_bounds__(kBlock) void k_view_index(int64_t *__restrict__ out
 // 8191 x 8189 Float32 takes 112-117 instead of 108.  Tiles of 64 x 64 measured
 // as well as 128 x 128 or better (small arrays: 4.5 us against 7.7); a side of
 // at most kNarrow elements takes tiles of 32 by 512 (8-byte: 128) instead
-// ([1000, 2000, 24] Float32 (0, 2, 1): 204 -> 79 us), and 8-byte copies of
-// few tiles 32 x 32.
+// ([1000, 2000, 24] Float32 (0, 2, 1): 204 -> 79 us).  8-byte copies take smaller
+// tiles while 64 x 64 are too few for the CUs: 32 x 32 below 700000 elements, 32
+// along A by 64 below 3 million (Float64, in 32 x 32, 32 x 64 and 64 x 64: 800 x 801
+// 4.3, 4.5 and 5.1 us, 1023 x 1025 5.4, 5.2 and 5.9, 1600 x 1601 8.4, 7.5 and 8.8,
+// 2000 x 1800 11.0, 10.6 and 10.3).
 struct TileArgs {
   int64_t na, nb;    // extents along A and B
   uint32_t ta, tb;   // tiles along A and B
@@ -627,8 +630,10 @@ int launch_tiled(const ph::Layout &L, int A, int B, void *dst, int64_t d_extent,
   constexpr int W = sizeof(E) == 8 ? 128 : 512;
   if (L.shape[A] <= kNarrow) return launch_tile<E, 32, W>(L, A, B, dst, d_extent, src);
   if (L.shape[B] <= kNarrow) return launch_tile<E, W, 32>(L, A, B, dst, d_extent, src);
-  if constexpr (sizeof(E) == 8)
-    if (ph::layout_count(L) < 128 * 64 * 64) return launch_tile<E, 32, 32>(L, A, B, dst, d_extent, src);
+  if constexpr (sizeof(E) == 8) {
+    if (ph::layout_count(L) < 700000) return launch_tile<E, 32, 32>(L, A, B, dst, d_extent, src);
+    if (ph::layout_count(L) < 3000000) return launch_tile<E, 32, 64>(L, A, B, dst, d_extent, src);
+  }
   return launch_tile<E, 64, 64>(L, A, B, dst, d_extent, src);
 }
 

@@ -42,6 +42,15 @@ def test_transpose_tile_edges(ph, dt):
         assert np.array_equal(x.view().permute(*order).to_narr().to_numpy(), h.transpose(order)), (shape, order)
 
 
+@pytest.mark.parametrize("dt", ["BF16", "F64"])
+def test_transposes_either_side_of_a_tile_size(ph, dt):
+    """Below and above 700000 and 3 million elements (8-byte tiles change
+    there), and 20 million and 32 tiles either way (tiles in patches)."""
+    for k, (a, b) in enumerate([(836, 837), (837, 837), (701, 1001), (1731, 1733), (1733, 1733), (2049, 10007)]):
+        h, x = _array(ph, dt, (a, b), k)
+        assert np.array_equal(x.view().permute(1, 0).to_narr().to_numpy(), h.T), (a, b)
+
+
 @pytest.mark.parametrize("dt", ["Bool", "BF16", "I32", "F64"])
 def test_rows_across_vectors(ph, dt):
     for k, (rows, cols) in enumerate([(40, 9), (33, 16), (50, 35), (7, 700), (300, 31), (3, 5003)]):
