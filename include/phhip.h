@@ -538,7 +538,8 @@ int ph_gbatch_destroy(void *handle);
 /* ---------------------------------------------------------------------------
  * Diagnostics (no reference counterpart).
  * ph_compile_check generates and compiles, without launching, the fused
- * kernels ph_map (kind 0) and ph_reduce2d_all (kind 1) would use for `prog`
+ * kernels ph_map (kind 0) and ph_reduce2d_all (kind 1; also those of a kept
+ * middle axis, for even cols) would use for `prog`
  * over contiguous inputs of the given dtypes and a rows x cols shape, and
  * (kind 2) the tiled map ph_map uses when input 0 is the transposed view of
  * a cols x rows array (rows and cols of 16 or more).  Kind 3 compiles the

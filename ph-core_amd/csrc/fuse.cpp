@@ -3274,26 +3274,43 @@ int ph_compile_check(const ph_prog *prog, int32_t n_in, const int32_t *in_dtypes
     V.cs[j] = 1;
     V.off[j] = 0;
   }
-  RedPlan P;
-  P.rows = rows;
-  P.cols = cols;
-  P.vec = 4;
-  P.do_cols = P.do_rows = P.do_full = true;
-  const int odt = prog->out_dtype;
-  if (odt == PH_I32 || odt == PH_BOOL) {
-    P.state = "SI"; P.state_bytes = sizeof(HostSI); P.acc_t = "i64";
-  } else {
-    P.state = "SF"; P.state_bytes = sizeof(HostSF); P.acc_t = "float";
+  // the reduction of a 2-D view (integer results: with bounds on the running
+  // totals, and exact), and per row over columns in two parts (a middle axis
+  // kept) where the columns halve
+  const bool ints = prog->out_dtype == PH_I32 || prog->out_dtype == PH_BOOL;
+  for (int form = 0; form < 4; ++form) {
+    const bool bounds = form & 1, two = form & 2;
+    if ((bounds && !ints) || (two && cols % 2 != 0)) continue;
+    RedPlan P;
+    P.rows = rows;
+    P.cols = cols;
+    P.do_rows = true;
+    P.do_cols = P.do_full = !two;
+    if (ints) {
+      P.state = "SI"; P.state_bytes = sizeof(HostSI); P.acc_t = "i64";
+    } else {
+      P.state = "SF"; P.state_bytes = sizeof(HostSF); P.acc_t = "float";
+    }
+    P.bounds = bounds;
+    P.vec = red_vec(ints && !bounds, n_in, in_dt);
+    if (two) P.cols2 = cols / 2;
+    for (int j = 0; j < PH_MAX_INPUTS; ++j) {
+      if (j < n_in && two) {
+        V.rs[j] = cols / 2;
+        P.cs2[j] = rows * (cols / 2);
+      }
+      P.vec_ok[j] = j < n_in && (two ? cols / 2 : cols) % P.vec == 0;
+    }
+    P.ntc = (cols + 256 * P.vec - 1) / (256 * P.vec);
+    P.ntc_fin = prefolded(P.ntc, kRowFold);
+    P.tr = 64;
+    P.ntr = (rows + 63) / 64;
+    P.ntr_fin = prefolded(P.ntr, kColFold);
+    P.parts = column_parts(P.ntr_fin, cols);
+    const int rc1 = ph::jit_compile_only(red_source(prog, n_in, in_dt, V.rs, V.cs, P));
+    if (rc1) return rc1;
   }
-  P.vec = red_vec(std::string(P.state) == "SI", n_in, in_dt);
-  for (int j = 0; j < PH_MAX_INPUTS; ++j) P.vec_ok[j] = j < n_in && cols % P.vec == 0;
-  P.ntc = (cols + 256 * P.vec - 1) / (256 * P.vec);
-  P.ntc_fin = prefolded(P.ntc, kRowFold);
-  P.tr = 64;
-  P.ntr = (rows + 63) / 64;
-  P.ntr_fin = prefolded(P.ntr, kColFold);
-  P.parts = column_parts(P.ntr_fin, cols);
-  return ph::jit_compile_only(red_source(prog, n_in, in_dt, V.rs, V.cs, P));
+  return PH_OK;
 }
 
 int ph_map_indexed(const ph_prog *prog, int32_t n_in, const void *const *ins, const ph_view_desc *in_descs,

@@ -281,6 +281,15 @@ def test_reduction_prefold_compiles_for_gfx950(host):
         host.compile_check(e, [d], 1 << 17, 64, 1)
 
 
+def test_reduction_forms_compile_for_gfx950(host):
+    """Every form of a reduction's kernels: integer results with bounds on
+    their running totals and exact, columns in one part and in two, tiles with
+    and without missing rows and columns, whole-vector and single loads."""
+    for d in (host.DType.I32, host.DType.F32, host.DType.BF16):
+        for rows, cols in [(128, 2048), (70, 1030)] if d != host.DType.BF16 else [(70, 1030)]:
+            host.compile_check(host.placeholder(d), [d], rows, cols, 1)
+
+
 def test_indexed_map_programs_compile_for_gfx950(host):
     """The kernels of a map whose source or destination is a view chain
     longer than one descriptor (operands addressed through index arrays:
