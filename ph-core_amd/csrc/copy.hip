@@ -109,7 +109,10 @@ __global__ __launch_bounds__(kBlock) void k_fill_rows(E *__restrict__ dst, E val
 // stays there for the kernel that reads it next.  Both ways, 8192^2 Int32: the
 // transposing copy 79 us streamed, 110 not; the gather of a strided view and
 // the fill+scatter that reads it 92 us streamed, 71 not (45 MB between them).
-// (A copy that nothing reads next is up to 2 us faster streamed below that.)
+// (Of a loop that gathers alone, a smaller source then stays there in
+// the destination's place: 5000^2 through every other column, 27 us streamed and
+// 32 not for Int32, 44 and 50 for Float64; with a sum of the result after each
+// gather 53 and 50, 87 and 82.)
 // The choice is a template argument: of a run-time one the compiler makes a
 // single store that is not streamed.
 bool streams(int64_t bytes) { return bytes > kStreamBytes; }
@@ -317,8 +320,8 @@ __global__ __launch_bounds__(kBlock) void k_view_index(int64_t *__restrict__ out
 // transposes them in registers and stores VW vectors along B into LDS [A][B].
 // The vector index within an LDS row is XOR-swizzled by (a / VW), so the lanes
 // of a store and of the read that follows touch distinct banks.  The tile
-// leaves LDS as vectors along B.  Either side moves whole runs of 512 bytes
-// (128 x 128 tiles of 4-byte elements), every element read once and written
+// leaves LDS as vectors along B.  Either side moves runs of a tile's edge (256
+// bytes in 64 x 64 tiles of 4-byte elements), every element read once and written
 // once; vectors need element alignment only, so odd extents and row pitches
 // run the same way, with single elements where a vector crosses the edge.
 //
@@ -564,7 +567,7 @@ Div32 make_div(int64_t d) {
 // Whether k_copy_flat_vec takes a copy: rows contiguous on both sides (the
 // source also backwards), and 31-bit addresses.
 bool flat_rows(const ph::Layout &L, const ph_view_desc *dd, const ph_view_desc *sd, int esize) {
-  if (L.rank < 1 || !fits_i32(dd, sd) || ph::layout_count(L) > INT32_MAX - 4096) return false;
+  if (L.rank < 1 || !fits_i32(dd, sd) || ph::layout_count(L) > INT32_MAX) return false;
   const int q = L.rank - 1;
   if (L.stride[0][q] != 1 || (L.stride[1][q] != 1 && L.stride[1][q] != -1)) return false;
   // Long rows of 8-byte elements into a strided destination: a wavefront's
@@ -694,8 +697,9 @@ int launch_copy(void *dst, const ph_view_desc *dd, const void *src, const ph_vie
   hipLaunchKernelGGL((k_copy_rows<E, EPT, I, D, S, NT>), grid, block, 0, st, (E *)dst, (const E *)src, a)
     const bool nt = streams(dd->extent * (int64_t)sizeof(E));
     if (small) {
-      if (dc && sc && nt) PH_COPY_LAUNCH(int32_t, true, true, true);
-      else if (dc && sc) PH_COPY_LAUNCH(int32_t, true, true, false);
+      constexpr bool both = sizeof(E) == 8;  // (flat_rows takes contiguous rows of smaller elements)
+      if (both && dc && sc && nt) PH_COPY_LAUNCH(int32_t, true, both, true);
+      else if (both && dc && sc) PH_COPY_LAUNCH(int32_t, true, both, false);
       else if (dc && nt) PH_COPY_LAUNCH(int32_t, true, false, true);
       else if (dc) PH_COPY_LAUNCH(int32_t, true, false, false);
       else if (sc) PH_COPY_LAUNCH(int32_t, false, true, false);
