@@ -300,10 +300,12 @@ bool cut(const Tile &t, int64_t ny, int64_t nx, int64_t k, Cut *c) {
 // to 10^6 columns and 20 others, 1 to 100 steps: on average within 3.7%
 // (Float32) and 2.7% (Float64) of the best tile and number of steps, and 16%
 // and 12% faster than with the first eight tiles alone.  A grid beyond the
-// 256 MB MALL is streamed: 5.6 TB/s (Float64) and 5.4 (Float32) at most, less in
-// tall tiles, in rows of 256 bytes and in few rows (8192^2, one step: Float64 195 us
-// in tiles of 4096 cells, 232 in 24576; Float32 101 us in 128 x 32, 114 in
-// 64 x 32, 121 in 128 x 24).
+// 256 MB MALL is streamed, at less in tall tiles, in rows of 256 bytes and in few
+// rows (8192^2, one step: Float64 195 us in tiles of 4096 cells, 232 in 24576;
+// Float32 101 us in 128 x 32, 114 in 64 x 32, 121 in 128 x 24); the Float32 rate
+// is lower than the best measured, 5.3 TB/s, since four steps hide behind it in
+// part only (109 us in 128 x 96 and 115 in 128 x 192, which the higher rate
+// preferred).
 struct Cost {
   double launch, fixed, alone, shared;  // a step alone: fixed + alone * work; with others: shared * work
 };
@@ -332,7 +334,7 @@ double pass_us(const Tile &t, int64_t ny, int64_t nx, int64_t k, const Cut &c) {
   const double cells = t.v * t.w * t.r / 16.0;  // of a tile, in 1024
   const bool few = t.w < 8 && c.nty > 1;
   const double stream = f64 ? bytes / 5.65e6 * (1 + 0.009 * cells) * (t.v == 1 ? 1.02 : 1) * (few ? 1.08 : 1)
-                            : bytes / 5.4e6 * (1 + 0.005 * cells) * (t.v == 1 ? 1.09 : 1) * (few ? 1.2 : 1);
+                            : bytes / 4.7e6 * (1 + 0.004 * cells) * (t.v == 1 ? 1.09 : 1) * (few ? 1.2 : 1);
   return std::max(us, stream);
 }
 
