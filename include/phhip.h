@@ -180,7 +180,8 @@ const char *ph_last_error(void);
 /* Device buffers backing an NArray (src/n_array.cr:20 `@buffer : Slice(T)`). */
 int ph_alloc(void **ptr, size_t bytes);
 int ph_free(void *ptr);
-/* Synchronous copies (the stream is drained first). */
+/* Synchronous copies (the stream is drained first).  Null pointers, and ranges
+ * that leave a buffer of ph_alloc, are PH_E_HIP. */
 int ph_h2d(void *dst, const void *src, size_t bytes);
 int ph_d2h(void *dst, const void *src, size_t bytes);
 /* Asynchronous device-to-device copy on the library stream. */
@@ -378,8 +379,8 @@ int ph_reduce2d_all(const ph_prog *prog, int32_t n_in, const void *const *ins,
  * is stated against the Float64 run.  u holds the initial field and
  * receives the final one; tmp is scratch of the same size.  Many steps
  * run per pass over the grid (tiles of it stay in registers meanwhile; a grid
- * of up to 64 x 64 cells runs them all in one launch), bit-identical to single
- * steps.  If
+ * that fits one tile runs up to 4096 of them, or those to the next energy, in one
+ * launch), bit-identical to single steps.  If
  * energy_every > 0, energy_out
  * (device, steps/energy_every + 1 doubles) receives the FP64 sum of u at
  * steps 0, energy_every, 2*energy_every, ...

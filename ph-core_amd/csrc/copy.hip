@@ -334,8 +334,9 @@ __global__ __launch_bounds__(kBlock) void k_view_index(int64_t *__restrict__ out
 // plain order); those deal patches of 2 x 8 tiles to the XCDs in turn (204).
 // Vectors and numbering together, against single elements in plain order:
 // [257, 1023, 515] Float32 permuted (2, 0, 1) 385 -> 221 us (4.9 TB/s),
-// 4096 x 4100 27 -> 21, 8192^2 89 -> 80; BFloat16 8192^2 82 -> 45.  An odd
-// 8191 x 8189 Float32 takes 112-117 instead of 108.  Tiles of 64 x 64 measured
+// 4096 x 4100 27 -> 21, 8192^2 89 -> 80, 8193 x 8195 140 -> 117 (8191 x 8189, whose
+// pitch falls the other way, 108 -> 115; patches of 8 x 2: 129 and 108); BFloat16
+// 8192^2 82 -> 45.  Tiles of 64 x 64 measured
 // as well as 128 x 128 or better (small arrays: 4.5 us against 7.7); a side of
 // at most kNarrow elements takes tiles of 32 by 512 (8-byte: 128) instead
 // ([1000, 2000, 24] Float32 (0, 2, 1): 204 -> 79 us).  8-byte copies take smaller
